@@ -40,29 +40,29 @@ def _quantize(name, n, k, layers, bs, col, zp, dtype):
 def listed():
     return [
         # one projection for one token: the smallest call there is, all latency
-        _layer("one projection, one token", 1, 4096, 4096, 1, 64, True, False, "float16", False),
+        _layer("one projection one token", 1, 4096, 4096, 1, 64, True, False, "float16", False),
         # one token of a conversation: every layer called once, weights from memory each time
-        _step("decode step, one token", 1, 4096, 11008, 128256, 2, 32, True, True, "float16"),
+        _step("decode step one token", 1, 4096, 11008, 128256, 2, 32, True, True, "float16"),
         # a dozen conversations decoded together in bfloat16
-        _step("decode step, 12 tokens, bf16", 12, 4096, 11008, 128256, 2, 64, True, True, "bfloat16"),
+        _step("decode step 12 tokens bf16", 12, 4096, 11008, 128256, 2, 64, True, True, "bfloat16"),
         # the widest layer of a large network at batch 16
         _layer("batch 16 on a wide layer", 16, 28672, 8192, 3, 64, True, True, "float16", False),
         # a loaded server between decoding and prompts; biased up-projections
-        _layer("batch 48, up-projection", 48, 11008, 4096, 8, 32, True, True, "float16", True),
+        _layer("batch 48 up-projection", 48, 11008, 4096, 8, 32, True, True, "float16", True),
         # weights quantized in blocks along N, an odd batch
-        _layer("batch 150, blocks along N", 150, 4096, 4096, 8, 32, False, True, "float16", False),
+        _layer("batch 150 blocks along N", 150, 4096, 4096, 8, 32, False, True, "float16", False),
         # a chunk of a prompt mixed with decoding
         _layer("chunk of 512", 512, 4096, 4096, 4, 64, True, True, "float16", True),
         # a prompt of no round length, bfloat16, without zero-points
-        _layer("prompt of 777, bf16", 777, 11008, 4096, 2, 64, True, False, "bfloat16", False),
+        _layer("prompt of 777 bf16", 777, 11008, 4096, 2, 64, True, False, "bfloat16", False),
         # a prompt of 2048 tokens through one projection
         _layer("prompt of 2048", 2048, 4096, 4096, 1, 64, True, True, "float16", False),
         # the largest product: a batch of prompts through the widest layer, the finest blocks
-        _layer("prompts of 4096, wide layer", 4096, 28672, 8192, 1, 16, True, True, "float16", False),
+        _layer("prompts of 4096 wide layer", 4096, 28672, 8192, 1, 16, True, True, "float16", False),
         # a network is loaded: the widest layer in the finest blocks
         _quantize("quantize a wide layer", 28672, 8192, 1, 16, True, True, "float16"),
         # and several ordinary layers in bfloat16, blocks along N
-        _quantize("quantize, bf16, along N", 11008, 4096, 4, 32, False, True, "bfloat16"),
+        _quantize("quantize bf16 along N", 11008, 4096, 4, 32, False, True, "bfloat16"),
     ]
 
 
