@@ -22,8 +22,11 @@
 
 namespace {
 
-constexpr int kTileN = 64;    // columns (n) per workgroup, blocks along N
-constexpr int kTileK = 256;   // rows (k) per workgroup
+constexpr int kTileK = 256;  // rows (k) per workgroup
+// Blocks along N: columns per workgroup.  64, but 32 for blocks of 32, whose kernel then needs 54 - 56 instead of 76 - 80
+// registers (8 waves a SIMD instead of 6): 4096 x 11008 bf16 with zero-points 24.6 -> 21.2 us, fp16 22.0 -> 20.7.  Blocks of
+// 16 stay level (fp16 23.6 | 24.8 and, 8192 x 28672, 107.7 | 105.0; bf16 25.3 | 25.8, 112.3 | 116.6), blocks of 64 need 64.
+constexpr int row_tile_n(int block_size) { return block_size == 32 ? 32 : 64; }
 // Blocks along K: 32 columns per workgroup, four 16-byte loads per lane.  A kernel that moves the same bytes the same
 // way and computes nothing was measured on K = 8192, N = 28672 with blocks of 16 for several tile shapes: 64 x 256
 // (eight loads per lane) 105.4 - 106.5 us, 32 x 256 103.6, 32 x 512 with 1 KiB per wave-load 105.7, 64 x 512 and 128 x 256
@@ -205,10 +208,8 @@ __device__ __forceinline__ BlockQuant block_quant(float mn, float mx) {
 
 // One weight: clamp(roundf(fmaf(v, reciprocal_scale, zp)), 0, 15) (reference: f16_quant_sm80.cuh:296-313); clamping
 // before rounding gives the same nibble as the reference's round-then-clamp (both are monotonic).
-template <bool BF>
 __device__ __forceinline__ uint32_t quantize_one(float v, float reciprocal_scale, float zp_f) {
-  const float r = __builtin_amdgcn_fmed3f(__fmaf_rn(v, reciprocal_scale, zp_f), 0.0f, 15.0f);
-  return BF ? round_0_to_15(r) : round_0_to_15_rpi(r);
+  return round_0_to_15_rpi(__builtin_amdgcn_fmed3f(__fmaf_rn(v, reciprocal_scale, zp_f), 0.0f, 15.0f));
 }
 
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
@@ -354,7 +355,7 @@ __global__ __launch_bounds__(kThreads) void prepack_kernel(const uint16_t* __res
       } else {
         v = static_cast<float>(__builtin_bit_cast(half2_t, words[t >> 1])[t & 1]);  // folded into the fma
       }
-      word |= quantize_one<BF>(v, b.reciprocal_scale, zp_f) << nibble_shift(t);
+      word |= quantize_one(v, b.reciprocal_scale, zp_f) << nibble_shift(t);
     }
 
     w_lds[kl >> 5][nl][(kl >> 3) & 3] = word;
@@ -416,14 +417,41 @@ __global__ __launch_bounds__(kThreads) void prepack_kernel(const uint16_t* __res
 // eight has its own scale and zero-point (reference: the [1, bs] block shape of
 // src/mickey/blk_q4/f16_quant_sm80.cuh:206-212, 225-315).  Same tile, same packed weight layout and
 // the same arithmetic as above; only the reduction runs across columns.  A wave covers 64 k of all
-// 64 columns of the tile: lane = (column & 7) * 8 + (k / 8), eight passes of 8 columns, so a block
+// columns of the tile: lane = (column & 7) * 8 + (k / 8), passes of 8 columns, so a block
 // is BS/8 passes times 8 lanes.
+//
+// Bound by vector instructions, so every block's scale is derived by ONE lane: the eight lanes of a block hold eight
+// minima and maxima each (one per k) and reduce them by halves -- the lanes 32 apart keep four k each, then 16 apart two,
+// then 8 apart one (permlane swaps and a row rotation, no LDS) -- after which the lane of column c has the range of its
+// k number c, derives scale, zero-point and reciprocal, stores the first two and hands reciprocal and zero-point to the
+// block's other lanes through a few hundred bytes of LDS that only its wave touches.  (When all eight lanes reduced all
+// eight k with ds_bpermute and derived all eight scales each: four 4096 x 11008 layers, blocks of 32 with zero-points,
+// bf16 132.7 us = 3.5 TB/s; so 88 us = 5.3 TB/s, as with blocks along K.)  The loads carry no branches: behind one each,
+// every load was waited for before the next was issued (fp16, the same layers one by one: 32 us, without 22).
 //
 // Scales and zero-points leave in the reference's packed order for this blocking
 // (f16_quant_sm80.cuh:506-512, 528-539): column-major [K][N/BS], and inside every group of 16
 // rows scale rows (2t, 2t+1, 2t+8, 2t+9) and zero-point rows (2t, 2t+8, 2t+1, 2t+9) sit at
 // positions 4t .. 4t+3.
 // ------------------------------------------------------------------------------------------------
+
+// The halving steps of the reduction: a holds the values of the lanes' first half of the rows, b of their second half;
+// afterwards the lower lanes have both lanes' a, the upper ones both lanes' b, ready to be combined.
+__device__ __forceinline__ void swap_32_apart(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+__device__ __forceinline__ void swap_16_apart(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+// a lane's value exchanged with lane ^ 8
+__device__ __forceinline__ uint32_t exchange_8_apart(uint32_t x) {
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x128 /* row_ror:8 */, 0xf, 0xf, true));
+}
+
 template <int BS, bool HAS_ZP, bool ALIGNED, bool BF = false>
 __global__ __launch_bounds__(kThreads) void prepack_rowwise_kernel(const uint16_t* __restrict__ src, int K,
                                                                    int N, int ld,
@@ -432,8 +460,12 @@ __global__ __launch_bounds__(kThreads) void prepack_rowwise_kernel(const uint16_
                                                                    uint8_t* __restrict__ zps, unsigned k_tiles,
                                                                    bool /*wide_meta*/) {
   constexpr int kPasses = BS / 8;            // passes of 8 columns that make up one block
-  constexpr int kGroups = kTileN / BS;       // blocks along N in one tile
-  __shared__ uint32_t w_lds[kTileK / 32][kTileN][4];
+  constexpr int kCols = row_tile_n(BS);      // columns of the tile
+  constexpr int kGroups = kCols / BS;        // blocks along N in one tile
+  constexpr int kLoads = kCols / 8;          // passes of the tile
+  __shared__ uint32_t w_lds[kTileK / 32][kCols][4];
+  // reciprocal of the scale and zero-point (as floats) of the 64 k of a wave, one block along N at a time
+  __shared__ __attribute__((aligned(16))) float q_lds[kThreads / 64][64][2];
 
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
@@ -441,63 +473,131 @@ __global__ __launch_bounds__(kThreads) void prepack_rowwise_kernel(const uint16_
   const int c8 = lane >> 3;  // column inside a pass
   const int kq = lane & 7;   // which 8 k of the wave's 64
   const int k0 = static_cast<int>(blockIdx.x % k_tiles) * kTileK;
-  const int n0 = static_cast<int>(blockIdx.x / k_tiles) * kTileN;
+  const int n0 = static_cast<int>(blockIdx.x / k_tiles) * kCols;
   const int kl = wave * 64 + kq * 8;  // this lane's first k inside the tile
   const bool k_ok = (k0 + kl) < K;    // K is a multiple of 64: a wave's 64 k are all in or all out
 
-  uint4 raw[8];
+  // all loads first, without branches: lanes past the end of the matrix read its last column or its last 8 k instead
+  // (N is a multiple of BS: a block is all in or all out; what such lanes compute is never stored)
+  uint4 raw[kLoads];
 #pragma unroll
-  for (int it = 0; it < 8; ++it) {
-    const int n = n0 + it * 8 + c8;
-    raw[it] = make_uint4(0, 0, 0, 0);
-    if (k_ok && n < N) {  // N is a multiple of BS: a block is all in or all out
-      const uint16_t* p = src + static_cast<size_t>(n) * ld + (k0 + kl);
-      if constexpr (ALIGNED) {
-        raw[it] = load_once_16(p);
-      } else {
-        uint32_t w[4];
+  for (int it = 0; it < kLoads; ++it) {
+    const uint16_t* p = src + static_cast<size_t>(min(n0 + it * 8 + c8, N - 1)) * ld + min(k0 + kl, K - 8);
+    if constexpr (ALIGNED) {
+      raw[it] = load_once_16(p);
+    } else {
+      uint32_t w[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) w[i] = static_cast<uint32_t>(p[2 * i]) | (static_cast<uint32_t>(p[2 * i + 1]) << 16);
-        raw[it] = make_uint4(w[0], w[1], w[2], w[3]);
-      }
+      for (int i = 0; i < 4; ++i) w[i] = static_cast<uint32_t>(p[2 * i]) | (static_cast<uint32_t>(p[2 * i + 1]) << 16);
+      raw[it] = make_uint4(w[0], w[1], w[2], w[3]);
     }
   }
-#define BLKQ4_VALUE(it_, t_) \
-  bits_to_float<BF>((((t_) >> 1) == 0 ? raw[it_].x : ((t_) >> 1) == 1 ? raw[it_].y : ((t_) >> 1) == 2 ? raw[it_].z : raw[it_].w) >> (16 * ((t_) & 1)) & 0xffffu)
+  auto word_of = [&](int it, int i) -> uint32_t { return i == 0 ? raw[it].x : i == 1 ? raw[it].y : i == 2 ? raw[it].z : raw[it].w; };
+  auto value = [&](int it, int t) -> float {
+    const uint32_t w = word_of(it, t >> 1);
+    if constexpr (BF) {
+      return __uint_as_float((t & 1) ? (w & 0xffff0000u) : (w << 16));
+    } else {
+      return static_cast<float>(__builtin_bit_cast(half2_t, w)[t & 1]);
+    }
+  };
 
 #pragma unroll
   for (int g = 0; g < kGroups; ++g) {
-    float rs[8], zf[8];
-    uint32_t sbits[8], zq[8];
+    // range of the block of k = k0 + 64 wave + 8 kq + c8, i.e. of this lane's k number c8
+    float mn, mx;
+    if constexpr (BF) {
+      float lo[8], hi[8];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      // range of the block of k = k0 + kl + t: the passes of this group, then the 8 column lanes
-      float mn = BLKQ4_VALUE(g * kPasses, t), mx = mn;
+      for (int t = 0; t < 8; ++t) {
+        lo[t] = hi[t] = value(g * kPasses, t);
 #pragma unroll
-      for (int q = 1; q < kPasses; ++q) {
-        const float v = BLKQ4_VALUE(g * kPasses + q, t);
-        mn = fminf(mn, v);
-        mx = fmaxf(mx, v);
-      }
-#pragma unroll
-      for (int mask = 8; mask < 64; mask <<= 1) {
-        mn = fminf(mn, __shfl_xor(mn, mask));
-        mx = fmaxf(mx, __shfl_xor(mx, mask));
-      }
-      BlockQuant b = block_quant<HAS_ZP, BF>(mn, mx);
-      if constexpr (!HAS_ZP) {
-        if (mn == 0.0f && mx == 0.0f) {
-          // all-zero block: the sign comes from the block's first weight (its first column, this k)
-          const uint32_t w0 = ((t >> 1) == 0 ? raw[g * kPasses].x : (t >> 1) == 1 ? raw[g * kPasses].y
-                               : (t >> 1) == 2 ? raw[g * kPasses].z : raw[g * kPasses].w) >> (16 * (t & 1));
-          const uint32_t first = __shfl(w0, kq);
-          b.scale_bits = ~first & 0x8000u;
+        for (int q = 1; q < kPasses; ++q) {
+          const float v = value(g * kPasses + q, t);
+          lo[t] = fminf(lo[t], v);
+          hi[t] = fmaxf(hi[t], v);
         }
       }
-      rs[t] = b.reciprocal_scale;
-      zf[t] = static_cast<float>(b.zp);
-      sbits[t] = b.scale_bits & 0xffffu;
-      zq[t] = b.zp;
+      auto fold = [](float& a, float& b, bool far, bool least) {
+        uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+        if (far) {
+          swap_32_apart(x, y);
+        } else {
+          swap_16_apart(x, y);
+        }
+        a = least ? fminf(__uint_as_float(x), __uint_as_float(y)) : fmaxf(__uint_as_float(x), __uint_as_float(y));
+      };
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        fold(lo[t], lo[t + 4], true, true);
+        fold(hi[t], hi[t + 4], true, false);
+      }
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        fold(lo[t], lo[t + 2], false, true);
+        fold(hi[t], hi[t + 2], false, false);
+      }
+      const bool odd = (c8 & 1) != 0;
+      mn = fminf(odd ? lo[1] : lo[0], __uint_as_float(exchange_8_apart(__float_as_uint(odd ? lo[0] : lo[1]))));
+      mx = fmaxf(odd ? hi[1] : hi[0], __uint_as_float(exchange_8_apart(__float_as_uint(odd ? hi[0] : hi[1]))));
+    } else {
+      // fp16: pairs of k as they lie in the words (comparisons are exact in any precision)
+      uint32_t lo[4], hi[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        lo[i] = hi[i] = word_of(g * kPasses, i);
+#pragma unroll
+        for (int q = 1; q < kPasses; ++q) {
+          lo[i] = pk_min_f16(lo[i], word_of(g * kPasses + q, i));
+          hi[i] = pk_max_f16(hi[i], word_of(g * kPasses + q, i));
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        swap_32_apart(lo[i], lo[i + 2]);
+        lo[i] = pk_min_f16(lo[i], lo[i + 2]);
+        swap_32_apart(hi[i], hi[i + 2]);
+        hi[i] = pk_max_f16(hi[i], hi[i + 2]);
+      }
+      swap_16_apart(lo[0], lo[1]);
+      lo[0] = pk_min_f16(lo[0], lo[1]);
+      swap_16_apart(hi[0], hi[1]);
+      hi[0] = pk_max_f16(hi[0], hi[1]);
+      lo[0] = pk_min_f16(lo[0], exchange_8_apart(lo[0]));
+      hi[0] = pk_max_f16(hi[0], exchange_8_apart(hi[0]));
+      const int half = 16 * (c8 & 1);
+      mn = half_bits_to_float((lo[0] >> half) & 0xffffu);
+      mx = half_bits_to_float((hi[0] >> half) & 0xffffu);
+    }
+    BlockQuant b = block_quant<HAS_ZP, BF>(mn, mx);
+    if constexpr (!HAS_ZP) {
+      // all-zero block: the sign comes from the block's first weight (its first column, this k); that weight is in the
+      // lane of column 0, whose word i is asked for by the lanes with c8 / 2 = i
+      uint32_t first = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t w = static_cast<uint32_t>(__shfl(static_cast<int>(word_of(g * kPasses, i)), kq));
+        if ((c8 >> 1) == i) first = w;
+      }
+      if (mn == 0.0f && mx == 0.0f) b.scale_bits = ~(first >> (16 * (c8 & 1))) & 0x8000u;
+    }
+    q_lds[wave][kq * 8 + c8][0] = b.reciprocal_scale;
+    q_lds[wave][kq * 8 + c8][1] = static_cast<float>(b.zp);
+    // scale and zero-point of this lane's block, at their place in the 16-row group
+    const int n_first = n0 + g * BS;
+    if (k_ok && n_first < N) {
+      const int row = k0 + kl + c8;
+      const size_t base = static_cast<size_t>(n_first / BS) * K + (row & ~15);
+      const int upper = (row >> 3) & 1, pair = (row & 7) >> 1, odd = row & 1;
+      scales[base + 4 * pair + 2 * upper + odd] = static_cast<uint16_t>(b.scale_bits);
+      if constexpr (HAS_ZP) zps[base + 4 * pair + 2 * odd + upper] = static_cast<uint8_t>(b.zp);
+    }
+    // (written and read by this wave alone: LDS operations of a wave complete in order)
+    float rs[8], zf[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      rs[t] = q_lds[wave][kq * 8 + t][0];
+      zf[t] = q_lds[wave][kq * 8 + t][1];
     }
 #pragma unroll
     for (int q = 0; q < kPasses; ++q) {
@@ -505,37 +605,19 @@ __global__ __launch_bounds__(kThreads) void prepack_rowwise_kernel(const uint16_
       uint32_t word = 0;
 #pragma unroll
       for (int t = 0; t < 8; ++t) {
-        word |= quantize_one<BF>(BLKQ4_VALUE(it, t), rs[t], zf[t]) << nibble_shift(t);
+        word |= quantize_one(value(it, t), rs[t], zf[t]) << nibble_shift(t);
       }
       w_lds[kl >> 5][it * 8 + c8][(kl >> 3) & 3] = word;
     }
-    // meta data of the group: one lane per 8 rows writes them
-    const int n_first = n0 + g * BS;
-    if (c8 == 0 && k_ok && n_first < N) {
-      const int row16 = (k0 + kl) & ~15;   // first row of the 16-row group
-      const int upper = ((k0 + kl) >> 3) & 1;  // this lane holds rows 8..15 of the group
-      const size_t base = static_cast<size_t>(n_first / BS) * K + row16;
-#pragma unroll
-      for (int tp = 0; tp < 4; ++tp) {
-        // rows (2tp, 2tp+1) of this lane's eight
-        const uint32_t pair = sbits[2 * tp] | (sbits[2 * tp + 1] << 16);
-        *reinterpret_cast<uint32_t*>(scales + base + 4 * tp + 2 * upper) = pair;
-        if constexpr (HAS_ZP) {
-          zps[base + 4 * tp + upper] = static_cast<uint8_t>(zq[2 * tp]);
-          zps[base + 4 * tp + upper + 2] = static_cast<uint8_t>(zq[2 * tp + 1]);
-        }
-      }
-    }
   }
-#undef BLKQ4_VALUE
   __syncthreads();
 
   // packed weights: one 16-byte unit per thread and pass, 1 KiB contiguous per wave
 #pragma unroll
-  for (int r = 0; r < (kTileK / 32) * kTileN / kThreads; ++r) {
+  for (int r = 0; r < (kTileK / 32) * kCols / kThreads; ++r) {
     const int u = tid + r * kThreads;
-    const int ksl = u / kTileN;
-    const int nl = u % kTileN;
+    const int ksl = u / kCols;
+    const int nl = u % kCols;
     const int k = k0 + ksl * 32;
     const int n = n0 + nl;
     if (k < K && n < N) {
@@ -613,7 +695,7 @@ __global__ __launch_bounds__(256) void repack_kernel(const uint8_t* __restrict__
 //   counts[1]  symmetric blocks: every finite fp16 extreme but zero (an all-zero block's scale is a sign rule of
 //              its own in the kernels);
 //   counts[2]  the rounding: every float in [0, 15] through v_cvt_rpi_i32_f32 against roundf and against the
-//              add-and-truncate form the bf16 quantizer uses;
+//              add-and-truncate form the definition uses;
 //   counts[3]  cases looked at (1 007 713 280 + 63 486 + 1 097 859 073).
 // counts[0..2] count disagreements: all three must be zero.
 // ------------------------------------------------------------------------------------------------
@@ -662,7 +744,7 @@ __global__ void quant_selfcheck_clear(unsigned long long* counts) {
 // launch's own status.
 template <int BS>
 int launch_prepack(const blkq4_prepack_args* a) {
-  const int tile_n = a->column_wise ? kColTileN : kTileN;
+  const int tile_n = a->column_wise ? kColTileN : row_tile_n(BS);
   const unsigned k_tiles = (a->rows + kTileK - 1) / kTileK;
   const dim3 grid(k_tiles * static_cast<unsigned>((a->columns + tile_n - 1) / tile_n));
   const bool aligned = (reinterpret_cast<uintptr_t>(a->src) & 15u) == 0 && (a->ld % 8) == 0;

@@ -98,6 +98,18 @@ def test_gaussian_rowwise(oracle, capi, device, bs, has_offsets, rows, columns):
     check_against_oracle(oracle, capi, device, bs, w, has_offsets, column_wise=False)
 
 
+@pytest.mark.parametrize("bs", [16, 32])
+@pytest.mark.parametrize("has_offsets", [True, False])
+@pytest.mark.parametrize("rows,columns", [(64, 32), (320, 96), (576, 160)])
+def test_rowwise_columns_that_do_not_fill_a_tile(oracle, capi, device, bs, has_offsets, rows, columns):
+    rng = np.random.default_rng(bs * 15485863 + rows * 31 + columns + has_offsets)
+    w = (rng.standard_normal((columns, rows)) * 0.02).astype(np.float16)
+    w[:, 5] = -0.0
+    w[0, 9] = -0.0
+    w[1:, 9] = 0.0
+    check_against_oracle(oracle, capi, device, bs, w, has_offsets, column_wise=False)
+
+
 @pytest.mark.parametrize("bs", [16, 32, 64])
 @pytest.mark.parametrize("has_offsets", [True, False])
 @pytest.mark.parametrize("rows,columns", [(64, 32), (192, 96), (320, 160), (576, 672), (1024, 1024)])
