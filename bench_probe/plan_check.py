@@ -56,7 +56,8 @@ def shapes():
 def candidate_plans(column_wise, m, n, k):
     plans = ["auto"]
     kt = k // 64
-    tile_shapes = [(2, 1, 1, 4, 4, 1), (4, 1, 1, 4, 4, 1), (4, 2, 1, 4, 4, 1), (8, 2, 1, 4, 0, 1)]
+    tile_shapes = [(2, 1, 1, 4, 4, 1), (4, 1, 1, 4, 4, 1), (4, 2, 1, 4, 4, 1), (8, 2, 1, 4, 0, 1),
+                   (5, 2, 1, 4, 0, 1), (6, 2, 1, 4, 0, 1)]
     if column_wise:
         tile_shapes.append((4, 1, 1, 1, 4, 4))
         if m <= 64:
@@ -67,7 +68,7 @@ def candidate_plans(column_wise, m, n, k):
             tiles = -(-m // (32 * rt * wm)) * -(-n // (32 * nt * wn))
             rem = tiles % 256 or tiles
             for parts in (1, 2, 3, 4):
-                if parts > 1 and (kw > 1 or rt == 1 or (rt == 2 and wn == 8) or rem * parts > 256 or kt // parts < 4):
+                if parts > 1 and (kw > 1 or rt in (1, 5, 6) or (rt == 2 and wn == 8) or rem * parts > 256 or kt // parts < 4):
                     continue
                 plans.append(f"tile {rt} {nt} {wm} {wn} {pw} {kw} {parts}")
                 # the tile order of whole rounds dealt to the XCDs in blocks (1, 2, 4 or 8 row bands)

@@ -494,7 +494,12 @@ inline long ceil_div(long a, long b) { return (a + b - 1) / b; }
 // (64 x 32, 128 x 32, 128 x 64 each) plus four producer waves that only issue copies, and 256 x 256 tiles of
 // four waves of 256 x 64 (every register of a SIMD belongs to the one wave, which leaves no room for producer
 // waves).  Larger tiles convert fewer weights per MFMA; smaller ones fill the chip with smaller problems.
-constexpr int kTileShapes[4][5] = {{2, 1, 1, 4, 4}, {4, 1, 1, 4, 4}, {4, 2, 1, 4, 4}, {8, 2, 1, 4, 0}};
+// Between the last two, 160 x 256 and 192 x 256 tiles of the same kind as 256 x 256, never split: for row counts that
+// 128-row tiles cover in a round and a bit and 256-row tiles with a third of the rows, or of the chip, idle (M = 777,
+// N = 11008, K = 4096: 215 tiles of 160 rows 67.0 us, 172 of 256 rows 88 - 90, 301 of 128 rows 99.6; bf16 65.7, 83.6 - 86.1,
+// 102.2; M = 320, N = 28672, K = 8192: 224 tiles 133.7, 336 of 128 rows 163.0 with the last 80 in 3 parts, 190.7 without).
+constexpr int kTileShapes[6][5] = {{2, 1, 1, 4, 4}, {4, 1, 1, 4, 4}, {4, 2, 1, 4, 4}, {5, 2, 1, 4, 0}, {6, 2, 1, 4, 0}, {8, 2, 1, 4, 0}};
+constexpr bool tile_has_split_form(int rt) { return rt != 5 && rt != 6; }
 
 // Arrival counters first (one per split tile), then the fp32 partial tiles of the split tiles.
 constexpr size_t kCounterBytes = 16 * 1024;  // room for 4096 split tiles
@@ -557,7 +562,8 @@ inline int xcd_rows_for(const TileShape& t, int m) {
 // Measured microseconds per 64-deep k tile of one workgroup when `busy` workgroups share the chip (fp16, blocks
 // of 64 along K, K = 4096 ... 14336, N = 4096 ... 28672): flat while half the compute units idle, then rising with the
 // load on the memory system and the clock the chip holds -- 64 x 128: 0.29 (<= 192 workgroups) to 0.33 (256),
-// 128 x 128: 0.32 (<= 128) to 0.51, 128 x 256: 0.65 (<= 128) to 0.89, 256 x 256: 1.07 (<= 128) to 1.63 --
+// 128 x 128: 0.32 (<= 128) to 0.51, 128 x 256: 0.65 (<= 128) to 0.89, 256 x 256: 1.07 (<= 128) to 1.63,
+// 160 x 256: 0.78 to 1.10, 192 x 256: 0.89 to 1.21 --
 // and what a workgroup spends outside its main loop.  (Refitted after the loops were unrolled and the tiles dealt to
 // the XCDs in blocks: 128 x 128 had been 0.37 to 0.575 and lost M = 384 ... 512 at K = 11008 to slower plans by 10 %.)
 struct TileCost {
@@ -568,7 +574,7 @@ struct TileCost {
 // weight, which counts where the conversion is what a workgroup waits for; measured against that form, every plan, a k
 // step takes, up to half a chip busy and on a full chip:
 //   bf16 (50 shapes, M = 128 ... 1024): 64 x 128 tiles 1.30 and 1.14 x, 128 x 128 1.30 and 1.12, 128 x 256 1.16 and 1.04,
-//     256 x 256 1.09 and 1.00; the 128 x 32 tiles whose waves split the k tile 0.99; the streaming kernel 1.06;
+//     256 x 256 1.09 and 1.00 (160 x 256 1.06 and 0.99, 192 x 256 likewise); the 128 x 32 tiles whose waves split the k tile 0.99; the streaming kernel 1.06;
 //   blocks along N (36 shapes, M = 128 ... 512): 1.24 and 1.15, 1.11 and 1.085, 1.02, 1.01 and 1.00;
 //   blocks of 16 (36 shapes): 1.16 and 1.13, 1.14 and 1.09, 1.11 and 1.06, 1.075 and 1.04 (blocks of 32: as 64).
 // Where several apply the factors multiply: bf16 with blocks of 16 measures 1.50 and 1.29, 1.39 and 1.20, 1.31 and 1.11,
@@ -583,13 +589,14 @@ inline int tile_cost_row(bool column_wise, bool bf16, int block_size) {
   return (bf16 ? kCostBf16 : 0) | (!column_wise ? kCostBlocksAlongN : 0) | (block_size == 16 ? kCostBlocksOf16 : 0);
 }
 inline TileCost tile_cost(const TileShape& t, int row = kCostPlain) {
-  // 64 x 128, 128 x 128, 128 x 256, 256 x 256
-  static constexpr TileCost kPlain[4] = {{0.29, 0.00065, 1.0, 192}, {0.32, 0.0015, 2.0, 128}, {0.65, 0.0019, 2.0, 128}, {1.07, 0.0044, 3.0, 128}};
+  // 64 x 128, 128 x 128, 128 x 256, 256 x 256, 160 x 256, 192 x 256
+  static constexpr TileCost kPlain[6] = {{0.29, 0.00065, 1.0, 192}, {0.32, 0.0015, 2.0, 128}, {0.65, 0.0019, 2.0, 128},
+                                         {1.07, 0.0044, 3.0, 128}, {0.78, 0.0025, 3.0, 128}, {0.89, 0.0025, 3.0, 128}};
   // factors on the k step of (up to flat_until workgroups, 256 workgroups) for bf16, blocks along N, blocks of 16
-  static constexpr double kFactor[3][4][2] = {{{1.30, 1.14}, {1.30, 1.12}, {1.16, 1.04}, {1.09, 1.00}},
-                                              {{1.24, 1.15}, {1.11, 1.085}, {1.02, 1.02}, {1.01, 1.00}},
-                                              {{1.16, 1.13}, {1.14, 1.09}, {1.11, 1.06}, {1.075, 1.04}}};
-  const int shape = t.rt == 8 ? 3 : (t.rt == 4 && t.nt == 2) ? 2 : t.rt == 4 ? 1 : (t.rt == 2 && t.wn == 4) ? 0 : -1;
+  static constexpr double kFactor[3][6][2] = {{{1.30, 1.14}, {1.30, 1.12}, {1.16, 1.04}, {1.09, 1.00}, {1.06, 0.99}, {1.06, 0.99}},
+                                              {{1.24, 1.15}, {1.11, 1.085}, {1.02, 1.02}, {1.01, 1.00}, {1.04, 1.03}, {1.03, 1.02}},
+                                              {{1.16, 1.13}, {1.14, 1.09}, {1.11, 1.06}, {1.075, 1.04}, {1.10, 1.055}, {1.08, 1.045}}};
+  const int shape = t.rt == 8 ? 3 : t.rt == 6 ? 5 : t.rt == 5 ? 4 : (t.rt == 4 && t.nt == 2) ? 2 : t.rt == 4 ? 1 : (t.rt == 2 && t.wn == 4) ? 0 : -1;
   if (shape < 0) return {0.55, 0.0, 0.0, 256};  // tiles of one row tile (up to 64 rows)
   TileCost c = kPlain[shape];
   if (row == kCostPlain) return c;
@@ -756,6 +763,7 @@ inline TileShape tile_plan(bool column_wise, int m, int n, int k, size_t workspa
     }
   }
   for (const auto& sh : kTileShapes) {
+    if (!tile_has_split_form(sh[0])) continue;
     TileShape t = shape(sh[0], sh[1], sh[2], sh[3], sh[4]);
     const int rem = t.tiles % kComputeUnits;
     if (rem == 0) continue;

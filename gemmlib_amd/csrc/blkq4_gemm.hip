@@ -871,7 +871,7 @@ __global__ __launch_bounds__(64 * (WM * WN * KW + PW))
         }
       }
 #pragma unroll
-      for (int it = 0; it < 32 * kPassTiles / kRowsPerStore; ++it) {
+      for (int it = 0; it < 32 * (RT - r0 < kPassTiles ? RT - r0 : kPassTiles) / kRowsPerStore; ++it) {  // (rows staged in this pass)
         const int row = it * kRowsPerStore + srow;  // inside the pass
         uint4 v = lds_read_16(region + srow * kRowBytes + chunk * 16, it * kRowsPerStore * kRowBytes);
         if (bias != nullptr) {
@@ -935,6 +935,8 @@ int launch_one(const blkq4_gemm_args* a) {
 // The tile shapes that exist, (RT, NT, WM, WN, PW): what blkq4::choose() may ask for.  Those with whole rows
 // of 32 or 64 (one row tile only) have no split form and no form for blocks along N.
 #define BLKQ4_TILE_SHAPES(X) X(8, 2, 1, 4, 0) X(8, 1, 1, 4, 4) X(4, 2, 1, 4, 4) X(4, 1, 1, 4, 4) X(2, 1, 1, 4, 4)
+// 160 and 192 rows: unsplit only (they exist to fill one round of workgroups better, see blkq4_choose.h)
+#define BLKQ4_TILE_SHAPES_UNSPLIT(X) X(5, 2, 1, 4, 0) X(6, 2, 1, 4, 0)
 #define BLKQ4_TILE_SHAPES_ONE_ROW_TILE(X) X(1, 1, 1, 4, 4) X(1, 1, 1, 8, 0) X(2, 1, 1, 8, 0)
 // (RT, NT) of the tiles whose four computing waves split the k tile (one tile per workgroup, four producer waves);
 // blocks along K, no split form
@@ -961,6 +963,13 @@ int launch_plan(const blkq4_gemm_args* a) {
               : launch_one<BS, HAS_ZP, RT_, NT_, WM_, WN_, PW_, true, false>(a);                        \
   }
   BLKQ4_TILE_SHAPES(BLKQ4_TRY)
+#undef BLKQ4_TRY
+#define BLKQ4_TRY(RT_, NT_, WM_, WN_, PW_)                                                              \
+  if (t.rt == RT_ && t.nt == NT_ && t.wm == WM_ && t.wn == WN_ && t.pw == PW_ && !sk) {                 \
+    return a->column_wise ? launch_one<BS, HAS_ZP, RT_, NT_, WM_, WN_, PW_, false, false>(a)            \
+                          : launch_one<BS, HAS_ZP, RT_, NT_, WM_, WN_, PW_, true, false>(a);            \
+  }
+  BLKQ4_TILE_SHAPES_UNSPLIT(BLKQ4_TRY)
 #undef BLKQ4_TRY
 #define BLKQ4_TRY(RT_, NT_, WM_, WN_, PW_)                                                              \
   if (t.rt == RT_ && t.nt == NT_ && t.wm == WM_ && t.wn == WN_ && t.pw == PW_ && a->column_wise && !sk) { \

@@ -13,6 +13,7 @@ import numpy as np
 import pytest
 import torch
 
+from bf16_util import bf16_kat, grid_activations_bf16
 from gpu_util import gemm_on_gpu, max_rel_err, quantize_on_gpu, to_dev, to_np
 
 pytestmark = pytest.mark.gpu
@@ -338,3 +339,44 @@ def test_every_plan_given_as_text_is_exact_on_reference_construction(oracle, cap
         capi.gemm_with_plan("decode 16 1 8 2", bs, True, m, n, k, a_dev, q_w, q_s, q_zp, out)   # K is not 16 slices
     with pytest.raises(capi.Blkq4Error, match="Kernel execution failed: invalid argument"):
         capi.gemm_with_plan("tile 4 1 1 4 4 1 1 3", bs, True, m, n, k, a_dev, q_w, q_s, q_zp, out)  # no such cut
+
+
+TALL = ["tile 5 2 1 4 0 1 1", "tile 6 2 1 4 0 1 1"]   # 160 x 256 and 192 x 256 tiles
+
+
+@pytest.mark.parametrize("bs,has_offsets,column_wise,m,n,k,plans", [
+    # one row, whole tiles, one row more than they hold; N that ends inside a tile; fewer k tiles than the ring has slots
+    (64, True, True, 1, 32, 64, TALL), (16, True, True, 160, 256, 128, TALL), (32, False, True, 161, 544, 192, TALL),
+    (64, True, True, 193, 800, 256, TALL), (16, False, True, 777, 1056, 320, TALL), (32, True, True, 384, 4128, 704, TALL),
+    (64, True, False, 161, 320, 64, TALL), (16, True, False, 193, 272 + 16, 192, TALL), (32, False, False, 777, 1056, 320, TALL),
+])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_tiles_of_five_and_six_row_tiles(oracle, capi, device, bs, has_offsets, column_wise, m, n, k, plans, bf16):
+    check_plans_exact(oracle, capi, device, bs, has_offsets, column_wise, m, n, k, plans, bf16)
+
+
+def check_plans_exact(oracle, capi, device, bs, has_offsets, column_wise, m, n, k, plans, bf16):
+    """the reference's exact construction (sums that a float holds): bit for bit, whatever the order of the sums"""
+    rng = np.random.default_rng(m * 7 + n + k + bs)
+    if bf16:
+        kat = bf16_kat(oracle, bs, k, n, has_offsets, seed=m + n + k, column_wise=column_wise)
+        a = grid_activations_bf16(oracle, rng, m, k)
+        ref = oracle.gemm(a, kat["weights"], bf16=True)
+    else:
+        kat = oracle.kat_generate(bs, column_wise, k, n, has_offsets)
+        a = grid_activations(rng, m, k)
+        ref = oracle.gemm(a, kat["weights"]).view(np.uint16)
+    dtype = torch.bfloat16 if bf16 else torch.float16
+    dev = lambda x: torch.from_numpy(x.view(np.int16).copy()).to(device).view(dtype)  # noqa: E731
+    w_elems, meta_elems = capi.quant_size(bs, column_wise, k, n)
+    q_w = torch.empty(w_elems, dtype=torch.uint8, device=device)
+    q_s = torch.empty(meta_elems, dtype=dtype, device=device)
+    q_zp = torch.empty(meta_elems, dtype=torch.uint8, device=device) if has_offsets else None
+    capi.quant(bs, column_wise, dev(kat["weights"]), q_w, q_s, q_zp, bf16=bf16)
+    a_dev = dev(a)
+    for plan in plans:
+        guarded = torch.full((m + 64, n), float("nan"), dtype=dtype, device=device)
+        capi.gemm_with_plan(plan, bs, column_wise, m, n, k, a_dev, q_w, q_s, q_zp, guarded[:m], bf16=bf16)
+        torch.cuda.synchronize()
+        assert np.array_equal(guarded[:m].view(torch.int16).cpu().numpy().view(np.uint16), ref), plan
+        assert torch.isnan(guarded[m:]).all(), f"{plan}: rows past the last one were written"
