@@ -435,6 +435,17 @@ __global__ __launch_bounds__(kThreads) void prepack_kernel(const uint16_t* __res
 // positions 4t .. 4t+3.
 // ------------------------------------------------------------------------------------------------
 
+// Minimum and maximum of two pairs of fp16.  Not the inline assembly of the kernel above: their results go into permlane
+// swaps, which must not read a register in the two wait states after a vector instruction wrote it, and the compiler
+// keeps that distance for instructions it knows, not for assembly.  (With the assembly four swaps of the 24 instantiations
+// were one wait state too close.)  It also quietens signalling NaNs first, so that they do not count, as any other NaN.
+__device__ __forceinline__ uint32_t minnum_f16x2(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(half2_t, a), __builtin_bit_cast(half2_t, b)));
+}
+__device__ __forceinline__ uint32_t maxnum_f16x2(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(half2_t, a), __builtin_bit_cast(half2_t, b)));
+}
+
 // The halving steps of the reduction: a holds the values of the lanes' first half of the rows, b of their second half;
 // afterwards the lower lanes have both lanes' a, the upper ones both lanes' b, ready to be combined.
 __device__ __forceinline__ void swap_32_apart(uint32_t& a, uint32_t& b) {
@@ -548,23 +559,23 @@ __global__ __launch_bounds__(kThreads) void prepack_rowwise_kernel(const uint16_
         lo[i] = hi[i] = word_of(g * kPasses, i);
 #pragma unroll
         for (int q = 1; q < kPasses; ++q) {
-          lo[i] = pk_min_f16(lo[i], word_of(g * kPasses + q, i));
-          hi[i] = pk_max_f16(hi[i], word_of(g * kPasses + q, i));
+          lo[i] = minnum_f16x2(lo[i], word_of(g * kPasses + q, i));
+          hi[i] = maxnum_f16x2(hi[i], word_of(g * kPasses + q, i));
         }
       }
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         swap_32_apart(lo[i], lo[i + 2]);
-        lo[i] = pk_min_f16(lo[i], lo[i + 2]);
+        lo[i] = minnum_f16x2(lo[i], lo[i + 2]);
         swap_32_apart(hi[i], hi[i + 2]);
-        hi[i] = pk_max_f16(hi[i], hi[i + 2]);
+        hi[i] = maxnum_f16x2(hi[i], hi[i + 2]);
       }
       swap_16_apart(lo[0], lo[1]);
-      lo[0] = pk_min_f16(lo[0], lo[1]);
+      lo[0] = minnum_f16x2(lo[0], lo[1]);
       swap_16_apart(hi[0], hi[1]);
-      hi[0] = pk_max_f16(hi[0], hi[1]);
-      lo[0] = pk_min_f16(lo[0], exchange_8_apart(lo[0]));
-      hi[0] = pk_max_f16(hi[0], exchange_8_apart(hi[0]));
+      hi[0] = maxnum_f16x2(hi[0], hi[1]);
+      lo[0] = minnum_f16x2(lo[0], exchange_8_apart(lo[0]));
+      hi[0] = maxnum_f16x2(hi[0], exchange_8_apart(hi[0]));
       const int half = 16 * (c8 & 1);
       mn = half_bits_to_float((lo[0] >> half) & 0xffffu);
       mx = half_bits_to_float((hi[0] >> half) & 0xffffu);
