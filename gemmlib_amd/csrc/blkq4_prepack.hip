@@ -463,6 +463,14 @@ __device__ __forceinline__ uint32_t exchange_8_apart(uint32_t x) {
   return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x128 /* row_ror:8 */, 0xf, 0xf, true));
 }
 
+// Between the lanes' writes to LDS and other lanes' reads of them inside one wave, and back.  The hardware completes a
+// wave's LDS operations in order; this holds the compiler to their order and costs no instruction.
+__device__ __forceinline__ void order_lds_within_wave() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <int BS, bool HAS_ZP, bool ALIGNED, bool BF = false>
 __global__ __launch_bounds__(kThreads) void prepack_rowwise_kernel(const uint16_t* __restrict__ src, int K,
                                                                    int N, int ld,
@@ -603,13 +611,15 @@ __global__ __launch_bounds__(kThreads) void prepack_rowwise_kernel(const uint16_
       scales[base + 4 * pair + 2 * upper + odd] = static_cast<uint16_t>(b.scale_bits);
       if constexpr (HAS_ZP) zps[base + 4 * pair + 2 * odd + upper] = static_cast<uint8_t>(b.zp);
     }
-    // (written and read by this wave alone: LDS operations of a wave complete in order)
+    // (written and read by this wave alone)
+    order_lds_within_wave();
     float rs[8], zf[8];
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
       rs[t] = q_lds[wave][kq * 8 + t][0];
       zf[t] = q_lds[wave][kq * 8 + t][1];
     }
+    order_lds_within_wave();
 #pragma unroll
     for (int q = 0; q < kPasses; ++q) {
       const int it = g * kPasses + q;

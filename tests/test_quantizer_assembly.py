@@ -2,7 +2,10 @@
 compiled to assembly with the library's own flags and read).
 
 A permlane swap must not read a vector register in the two wait states after a vector instruction wrote it, and neither
-must an operand read through DPP.  The compiler keeps that distance for the instructions it knows and not for inline assembly."""
+must an operand read through DPP.  The compiler keeps that distance for the instructions it knows and not for inline assembly.
+
+Where lanes of a wave hand each other values through LDS, the source has to demand the order of the writes and the reads;
+a wave barrier (no instruction, a comment in the assembly) shows that it does."""
 
 import os
 import re
@@ -78,6 +81,16 @@ def test_cross_lane_instructions_keep_their_distance_from_what_they_read(kernels
         assert any("v_permlane32_swap" in line for line in kernels[name]), name
     bad = {name: pairs for name, lines in kernels.items() if (pairs := _too_close(lines))}
     assert not bad, bad
+
+
+@pytest.mark.parametrize("bs", [16, 32, 64])
+def test_values_handed_over_inside_a_wave_are_ordered_by_the_source(kernels, bs):
+    """blocks along N: one hand-over of reciprocals and zero-points per block of the tile, ordered on both sides"""
+    blocks = {16: 4, 32: 1, 64: 1}[bs]   # of a tile: 64 / 16, 32 / 32 and 64 / 64 columns
+    names = [k for k in kernels if f"rowwise_kernelILi{bs}E" in k]
+    assert len(names) == 8
+    for name in names:
+        assert sum("wave barrier" in line for line in kernels[name]) == 2 * blocks, name
 
 
 def test_the_distance_check_sees_what_it_is_meant_to_see():
