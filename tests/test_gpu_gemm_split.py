@@ -25,7 +25,23 @@ SPLIT_CASES = [
     # 33 to 64 rows: every 64 x 128 tile in parts, where the kernel would otherwise stream the weights
     (64, True, True, 64, 5120, 5120, "64 x 128", 4),
     (32, True, False, 40, 13824, 5120, "64 x 128", 2),
+    # 128 x 256 tiles in three parts: all of them (66), and what two whole rounds leave (52 of 564)
+    (32, False, True, 150, 8448, 11008, "128 x 256", 3),
+    (64, True, False, 650, 24064, 4096, "128 x 256", 3),
 ]
+# 300 rows are two 160-row tiles, which now cover this layer in one round, unsplit: the split is asked for by its text
+PLAN_AS_TEXT = {(300, 28672, 8192): "tile 4 2 1 4 4 1 3"}
+
+
+def _multiply(capi, device, bs, col, a, q_w, q_s, q_zp, n):
+    """the product with the split plan of the shape, the library's own choice or the one given as text"""
+    m, k = a.shape
+    if (m, n, k) not in PLAN_AS_TEXT:
+        return gemm_on_gpu(capi, device, bs, a, q_w, q_s, q_zp, n, column_wise=col)
+    out = torch.full((m, n), float("nan"), dtype=torch.float16, device=device)
+    capi.gemm_with_plan(PLAN_AS_TEXT[m, n, k], bs, col, m, n, k, to_dev(a, device), q_w, q_s, q_zp, out)
+    torch.cuda.synchronize()
+    return to_np(out)
 
 
 def _assert_split_plan(capi, bs, col, m, n, k, tile, parts, bf16=False):
@@ -35,7 +51,8 @@ def _assert_split_plan(capi, bs, col, m, n, k, tile, parts, bf16=False):
 
 @pytest.mark.parametrize("bs,col,has_offsets,m,n,k,tile,parts", SPLIT_CASES)
 def test_split_tiles_exact_on_reference_construction(oracle, capi, device, bs, col, has_offsets, m, n, k, tile, parts):
-    _assert_split_plan(capi, bs, col, m, n, k, tile, parts)
+    if (m, n, k) not in PLAN_AS_TEXT:
+        _assert_split_plan(capi, bs, col, m, n, k, tile, parts)
     rng = np.random.default_rng(m + n + k)
     kat = oracle.kat_generate(bs, col, k, n, has_offsets)
     a = grid_activations(rng, m, k)
@@ -43,26 +60,30 @@ def test_split_tiles_exact_on_reference_construction(oracle, capi, device, bs, c
     assert np.array_equal(to_np(q_w), oracle.native_from_canonical(kat["canon_w"]))
     ref = oracle.gemm(a, kat["weights"])
     for call in range(3):  # the workspace and its counters are used again by every call
-        got = gemm_on_gpu(capi, device, bs, a, q_w, q_s, q_zp, n, column_wise=col)
+        got = _multiply(capi, device, bs, col, a, q_w, q_s, q_zp, n)
         bad = np.argwhere(got.view(np.uint16) != ref.view(np.uint16))
         assert bad.shape[0] == 0, f"call {call}: {bad.shape[0]} of {m * n} outputs differ, first {bad[:5].tolist()}"
 
 
-@pytest.mark.parametrize("bs,col,has_offsets,m,n,k,tile,parts", SPLIT_CASES[:6:2] + SPLIT_CASES[6:7] + SPLIT_CASES[8:9])
+@pytest.mark.parametrize("bs,col,has_offsets,m,n,k,tile,parts", SPLIT_CASES[:6:2] + SPLIT_CASES[6:7] + SPLIT_CASES[8:9] + SPLIT_CASES[10:])
 def test_split_tiles_gaussian_deterministic_and_with_bias(oracle, capi, device, bs, col, has_offsets, m, n, k, tile, parts):
+    if (m, n, k) not in PLAN_AS_TEXT:
+        _assert_split_plan(capi, bs, col, m, n, k, tile, parts)
     a, w = gaussian_problem(7 * m + n + k, m, n, k)
     q_w, q_s, q_zp = quantize_on_gpu(capi, device, bs, w, has_offsets, column_wise=col)
     canon, s, z = oracle.quantize(bs, col, w, has_offsets)
     b = oracle.dequantize(bs, col, canon, s, z)
     rows = np.unique(np.linspace(0, m - 1, 24).astype(np.int64))
     ref = oracle.gemm(np.ascontiguousarray(a[rows]), b)
-    got = gemm_on_gpu(capi, device, bs, a, q_w, q_s, q_zp, n, column_wise=col)
+    got = _multiply(capi, device, bs, col, a, q_w, q_s, q_zp, n)
     assert max_rel_err(got[rows], ref) <= 1e-2
     # the parts are added in a fixed order, whichever workgroup arrives last: every call gives the same bits
     for _ in range(4):
-        again = gemm_on_gpu(capi, device, bs, a, q_w, q_s, q_zp, n, column_wise=col)
+        again = _multiply(capi, device, bs, col, a, q_w, q_s, q_zp, n)
         assert np.array_equal(again.view(np.uint16), got.view(np.uint16))
     # bias in the epilogue of the workgroup that finishes the tile: fp16 result + fp16 bias, rounded again
+    if (m, n, k) in PLAN_AS_TEXT:   # (a plan given as text takes no bias: the library's own plan against itself)
+        got = gemm_on_gpu(capi, device, bs, a, q_w, q_s, q_zp, n, column_wise=col)
     bias = torch.randn(n, generator=torch.Generator().manual_seed(3)).to(torch.float16)
     out = torch.empty(m, n, dtype=torch.float16, device=device)
     capi.gemm(bs, col, m, n, k, to_dev(a, device), q_w, q_s, q_zp, out, bias=bias.to(device))
