@@ -355,8 +355,9 @@ def test_tiles_of_five_and_six_row_tiles(oracle, capi, device, bs, has_offsets, 
     check_plans_exact(oracle, capi, device, bs, has_offsets, column_wise, m, n, k, plans, bf16)
 
 
-def check_plans_exact(oracle, capi, device, bs, has_offsets, column_wise, m, n, k, plans, bf16):
-    """the reference's exact construction (sums that a float holds): bit for bit, whatever the order of the sums"""
+def exact_problem(oracle, capi, device, bs, has_offsets, column_wise, m, n, k, bf16):
+    """the reference's exact construction (sums that a float holds: the same bits whatever the order of the sums)
+    -> activations, packed weights, scales and zero-points on the device, the product's bits"""
     rng = np.random.default_rng(m * 7 + n + k + bs)
     if bf16:
         kat = bf16_kat(oracle, bs, k, n, has_offsets, seed=m + n + k, column_wise=column_wise)
@@ -373,10 +374,39 @@ def check_plans_exact(oracle, capi, device, bs, has_offsets, column_wise, m, n, 
     q_s = torch.empty(meta_elems, dtype=dtype, device=device)
     q_zp = torch.empty(meta_elems, dtype=torch.uint8, device=device) if has_offsets else None
     capi.quant(bs, column_wise, dev(kat["weights"]), q_w, q_s, q_zp, bf16=bf16)
-    a_dev = dev(a)
+    return dev(a), q_w, q_s, q_zp, ref
+
+
+def bits_of(t):
+    return t.view(torch.int16).cpu().numpy().view(np.uint16)
+
+
+def check_plans_exact(oracle, capi, device, bs, has_offsets, column_wise, m, n, k, plans, bf16):
+    a_dev, q_w, q_s, q_zp, ref = exact_problem(oracle, capi, device, bs, has_offsets, column_wise, m, n, k, bf16)
     for plan in plans:
-        guarded = torch.full((m + 64, n), float("nan"), dtype=dtype, device=device)
+        guarded = torch.full((m + 64, n), float("nan"), dtype=a_dev.dtype, device=device)
         capi.gemm_with_plan(plan, bs, column_wise, m, n, k, a_dev, q_w, q_s, q_zp, guarded[:m], bf16=bf16)
         torch.cuda.synchronize()
-        assert np.array_equal(guarded[:m].view(torch.int16).cpu().numpy().view(np.uint16), ref), plan
+        assert np.array_equal(bits_of(guarded[:m]), ref), plan
         assert torch.isnan(guarded[m:]).all(), f"{plan}: rows past the last one were written"
+
+
+# the last tile's rows and columns are partly there; the second pass of the epilogue holds one row tile or two
+@pytest.mark.parametrize("bs,has_offsets,column_wise,m,n,k,tile", [
+    (64, True, True, 300, 25312, 192, "160 x 256"), (16, False, True, 300, 25312, 128, "160 x 256"),
+    (32, True, True, 333, 23200, 192, "192 x 256"), (16, True, True, 333, 22144, 128, "192 x 256"),
+    (64, True, False, 300, 26368, 128, "160 x 256"), (32, False, False, 333, 23232, 192, "192 x 256"),
+])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_five_and_six_row_tiles_as_the_library_chooses_them_and_with_bias(oracle, capi, device, bs, has_offsets, column_wise, m, n,
+                                                                          k, tile, bf16):
+    assert capi.gemm_plan(bs, column_wise, m, n, k, has_offsets, bf16)[2].startswith(f"tile: {tile},")
+    a_dev, q_w, q_s, q_zp, ref = exact_problem(oracle, capi, device, bs, has_offsets, column_wise, m, n, k, bf16)
+    bias = (torch.randn(n, generator=torch.Generator().manual_seed(n)) * 0.5).to(a_dev.dtype).to(device)
+    for b in (None, bias):
+        guarded = torch.full((m + 64, n), float("nan"), dtype=a_dev.dtype, device=device)
+        capi.gemm(bs, column_wise, m, n, k, a_dev, q_w, q_s, q_zp, guarded[:m], bias=b, bf16=bf16)
+        torch.cuda.synchronize()
+        want = torch.from_numpy(ref.view(np.int16).copy()).to(device).view(a_dev.dtype)
+        assert np.array_equal(bits_of(guarded[:m]), bits_of(want if b is None else want + b))   # (rounded before and after)
+        assert torch.isnan(guarded[m:]).all(), "rows past the last one were written"
