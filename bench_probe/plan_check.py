@@ -34,7 +34,9 @@ VARIANTS = {
 FITTED_VARIANTS = {"fp16/bs64": (False, 64, True, True), "fp16/bs64/sym": (False, 64, True, False),
                    # combinations, for --shapes
                    "bf16/bs16": (True, 16, True, True), "bf16/bs64/along-N": (True, 64, False, True),
-                   "fp16/bs16/along-N": (False, 16, False, True), "fp16/bs32": (False, 32, True, True)}
+                   "fp16/bs16/along-N": (False, 16, False, True), "fp16/bs32": (False, 32, True, True),
+                   "bf16/bs16/along-N": (True, 16, False, True), "fp16/bs32/along-N": (False, 32, False, True),
+                   "bf16/bs32/along-N": (True, 32, False, True), "bf16/bs32": (True, 32, True, True)}
 LAYERS = [(4096, 4096), (11008, 4096), (4096, 11008), (28672, 8192), (14336, 4096)]   # (N, K)
 ROWS = [1, 4, 8, 16, 32, 64, 128, 256, 512]
 

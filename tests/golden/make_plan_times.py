@@ -7,6 +7,8 @@ form as blkq4_gemm_with_plan_sm80 takes it.  Plans more than 1.6 times slower th
 tests/test_kernel_choice.py holds the kernel choice against these times on the CPU.
 
     python3 tests/golden/make_plan_times.py times.jsonl [more.jsonl ...]
+
+A path that ends in .json is an earlier record: its shapes are kept in front of the new ones.
 """
 
 import json
@@ -15,12 +17,18 @@ import sys
 
 VARIANTS = {"fp16/bs64": (False, 64, True, True), "bf16/bs64": (True, 64, True, True), "fp16/bs16": (False, 16, True, True),
             "fp16/bs32/sym": (False, 32, True, False), "fp16/bs64/along-N": (False, 64, False, True),
-            "bf16/bs16": (True, 16, True, True), "bf16/bs64/along-N": (True, 64, False, True)}
+            "bf16/bs16": (True, 16, True, True), "bf16/bs64/along-N": (True, 64, False, True),
+            "fp16/bs16/along-N": (False, 16, False, True), "bf16/bs16/along-N": (True, 16, False, True),
+            "fp16/bs32/along-N": (False, 32, False, True), "bf16/bs32/along-N": (True, 32, False, True),
+            "fp16/bs32": (False, 32, True, True), "bf16/bs32": (True, 32, True, True)}
 
 
 def main(paths):
     rows = []
     for path in paths:
+        if path.endswith(".json"):
+            rows += json.load(open(path))
+            continue
         for line in open(path):
             try:
                 r = json.loads(line)
