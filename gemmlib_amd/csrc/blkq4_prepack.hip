@@ -588,17 +588,22 @@ __global__ __launch_bounds__(kThreads) void prepack_rowwise_kernel(const uint16_
       mn = half_bits_to_float((lo[0] >> half) & 0xffffu);
       mx = half_bits_to_float((hi[0] >> half) & 0xffffu);
     }
-    BlockQuant b = block_quant<HAS_ZP, BF>(mn, mx);
+    uint32_t first = 0;
     if constexpr (!HAS_ZP) {
-      // all-zero block: the sign comes from the block's first weight (its first column, this k); that weight is in the
-      // lane of column 0, whose word i is asked for by the lanes with c8 / 2 = i
-      uint32_t first = 0;
+      // the block's first weight (its first column, this k) decides what its extremes leave open; it is in the lane of
+      // column 0, whose word i is asked for by the lanes with c8 / 2 = i
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const uint32_t w = static_cast<uint32_t>(__shfl(static_cast<int>(word_of(g * kPasses, i)), kq));
         if ((c8 >> 1) == i) first = w;
       }
-      if (mn == 0.0f && mx == 0.0f) b.scale_bits = ~(first >> (16 * (c8 & 1))) & 0x8000u;
+      first = (first >> (16 * (c8 & 1))) & 0xffffu;
+      // a block without any number: the scale is the NaN of the first weight, not of whichever lane the halving ended with
+      if (mn != mn) mn = mx = bits_to_float<BF>(first);
+    }
+    BlockQuant b = block_quant<HAS_ZP, BF>(mn, mx);
+    if constexpr (!HAS_ZP) {
+      if (mn == 0.0f && mx == 0.0f) b.scale_bits = ~first & 0x8000u;  // all-zero block: its sign
     }
     q_lds[wave][kq * 8 + c8][0] = b.reciprocal_scale;
     q_lds[wave][kq * 8 + c8][1] = static_cast<float>(b.zp);

@@ -101,3 +101,25 @@ def test_weights_that_are_no_numbers(oracle, capi, device, bs, kind, has_offsets
     for k in range(320):   # one per block of a k at most, at every place of a block in turn, of both signs
         bits[(7 * k) % bs + bs * (k % (192 // bs)), k] = value | (0x8000 if k % 3 == 0 else 0)
     check(oracle, capi, device, bs, bits, has_offsets, bf16)
+
+
+@TYPES
+@BLOCKS
+@pytest.mark.parametrize("signalling", [False, True])
+def test_blocks_without_any_number_scale_by_their_first_weight(capi, device, bs, signalling, bf16):
+    """without zero-points: the scale is the first weight's NaN, made quiet, with its sign and payload"""
+    n, k = 192, 320
+    infinite, quiet = (0x7f80, 0x40) if bf16 else (0x7c00, 0x200)
+    rng = np.random.default_rng(bs)
+    bits = (infinite | (0 if signalling else quiet) | rng.integers(1, quiet, (n, k)) | (rng.integers(0, 2, (n, k)) << 15)).astype(np.uint16)
+    dtype = torch.bfloat16 if bf16 else torch.float16
+    w_elems, meta_elems = capi.quant_size(bs, False, k, n)
+    q_w = torch.full((w_elems,), 0xA5, dtype=torch.uint8, device=device)
+    q_s = torch.zeros(meta_elems, dtype=dtype, device=device)
+    capi.quant(bs, False, torch.from_numpy(bits.view(np.int16)).to(device).view(dtype), q_w, q_s, None, bf16=bf16)
+    torch.cuda.synchronize()
+    # packed order of the scales: inside 16 rows, rows 2t, 2t + 1, 2t + 8, 2t + 9 at 4t .. 4t + 3
+    order = [r for t in range(4) for r in (2 * t, 2 * t + 1, 2 * t + 8, 2 * t + 9)]
+    want = (bits[::bs] | quiet).reshape(n // bs, k // 16, 16)[:, :, order].reshape(-1)
+    assert np.array_equal(q_s.view(torch.int16).cpu().numpy().view(np.uint16), want)
+    assert not q_w.cpu().numpy().any()   # a weight that is no number becomes the nibble 0
