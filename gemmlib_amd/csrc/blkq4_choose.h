@@ -496,8 +496,9 @@ inline long ceil_div(long a, long b) { return (a + b - 1) / b; }
 // waves).  Larger tiles convert fewer weights per MFMA; smaller ones fill the chip with smaller problems.
 // Between the last two, 160 x 256 and 192 x 256 tiles of the same kind as 256 x 256, never split: for row counts that
 // 128-row tiles cover in a round and a bit and 256-row tiles with a third of the rows, or of the chip, idle (M = 777,
-// N = 11008, K = 4096: 215 tiles of 160 rows 67.0 us, 172 of 256 rows 88 - 90, 301 of 128 rows 99.6; bf16 65.7, 83.6 - 86.1,
-// 102.2; M = 320, N = 28672, K = 8192: 224 tiles 133.7, 336 of 128 rows 163.0 with the last 80 in 3 parts, 190.7 without).
+// N = 11008, K = 4096: 215 tiles of 160 rows 66.4 us, 172 of 256 rows, which it replaced, 79.1, 301 of 128 rows with the
+// last 45 in parts 87.0; bf16 67.0, 79.4, 87.6; M = 320, N = 28672, K = 8192: 224 tiles 129.2, 336 of 128 rows with the last
+// 80 in 3 parts, which it replaced, 158.7).
 constexpr int kTileShapes[6][5] = {{2, 1, 1, 4, 4}, {4, 1, 1, 4, 4}, {4, 2, 1, 4, 4}, {5, 2, 1, 4, 0}, {6, 2, 1, 4, 0}, {8, 2, 1, 4, 0}};
 constexpr bool tile_has_split_form(int rt) { return rt != 5 && rt != 6; }
 

@@ -23,9 +23,10 @@
 namespace {
 
 constexpr int kTileK = 256;  // rows (k) per workgroup
-// Blocks along N: columns per workgroup.  64, but 32 for blocks of 32, whose kernel then needs 54 - 56 instead of 76 - 80
-// registers (8 waves a SIMD instead of 6): 4096 x 11008 bf16 with zero-points 24.6 -> 21.2 us, fp16 22.0 -> 20.7.  Blocks of
-// 16 stay level (fp16 23.6 | 24.8 and, 8192 x 28672, 107.7 | 105.0; bf16 25.3 | 25.8, 112.3 | 116.6), blocks of 64 need 64.
+// Blocks along N: columns per workgroup.  64, but 32 for blocks of 32, whose bf16 kernel then needs 56 - 60 instead of
+// 74 - 76 registers (8 waves a SIMD instead of 6; fp16 39 - 43 instead of 62 - 64): 4096 x 11008 bf16 with zero-points
+// 24.6 -> 21.2 us, fp16 22.0 -> 20.7.  Blocks of 16 stay level (fp16 23.6 | 24.8 and, 8192 x 28672, 107.7 | 105.0; bf16
+// 25.3 | 25.8, 112.3 | 116.6), blocks of 64 need 64.
 constexpr int row_tile_n(int block_size) { return block_size == 32 ? 32 : 64; }
 // Blocks along K: 32 columns per workgroup, four 16-byte loads per lane.  A kernel that moves the same bytes the same
 // way and computes nothing was measured on K = 8192, N = 28672 with blocks of 16 for several tile shapes: 64 x 256
@@ -426,7 +427,7 @@ __global__ __launch_bounds__(kThreads) void prepack_kernel(const uint16_t* __res
 // k number c, derives scale, zero-point and reciprocal, stores the first two and hands reciprocal and zero-point to the
 // block's other lanes through a few hundred bytes of LDS that only its wave touches.  (When all eight lanes reduced all
 // eight k with ds_bpermute and derived all eight scales each: four 4096 x 11008 layers, blocks of 32 with zero-points,
-// bf16 132.7 us = 3.5 TB/s; so 88 us = 5.3 TB/s, as with blocks along K.)  The loads carry no branches: behind one each,
+// bf16 132.2 us = 3.5 TB/s; so 89.1 us = 5.2 TB/s, as with blocks along K.)  The loads carry no branches: behind one each,
 // every load was waited for before the next was issued (fp16, the same layers one by one: 32 us, without 22).
 //
 // Scales and zero-points leave in the reference's packed order for this blocking
@@ -803,7 +804,7 @@ int launch_prepack(const blkq4_prepack_args* a) {
 
 extern "C" int blkq4_dev_prepack(const blkq4_prepack_args* a) {
   if ((reinterpret_cast<uintptr_t>(a->packed_w) & 15u) != 0) return static_cast<int>(hipErrorInvalidValue);
-  // row-wise blocking: scale pairs are stored as 32-bit words; a block may not straddle the tile edge
+  // row-wise blocking: the GEMM kernels read these scales in pairs, as 32-bit words; a block may not straddle the tile edge
   if (!a->column_wise && ((reinterpret_cast<uintptr_t>(a->scales) & 3u) != 0 || (a->columns % a->block_size) != 0)) {
     return static_cast<int>(hipErrorInvalidValue);
   }
