@@ -5,7 +5,8 @@
 
 One "step" is one call of ``blkq4_fp16_gemm_sm80`` on the headline workload (C4: the M=2048 prefill
 GEMM); the GEMV (C2) and the other configurations are measured the same way and reported inside the
-same JSON line.  Inputs are resident in HBM before the timed region.  HBM-bound configurations rotate
+same JSON line by kernel time, roofline fraction and parity, and in full as a JSON object on stderr (the line with all of it
+had grown to 20 KB, which a reader that keeps the last 8 KB of the output cannot parse).  Inputs are resident in HBM before the timed region.  HBM-bound configurations rotate
 over distinct weight sets whose total size is at least twice the 256 MB Infinity Cache, and the timed
 graph visits every set equally often whatever ``--steps`` is.  Every configuration is replayed untimed
 until the clocks have settled.  Kernel time comes from HIP events on the launch stream around a captured
@@ -644,9 +645,8 @@ def main(argv=None) -> int:
         for key, ctx in (("C4", "library_fp16_gemm_c4_shape"), ("C5", "library_fp16_gemm_c5_shape")):
             if key in by_workload and ctx in line["context"]:
                 by_workload[key]["library_fp16_gemm_us"] = line["context"][ctx]["us"]
-    # the configurations the metric is defined on go last, so that they are what the end of the output shows
-    last = [k for k in ("C1", "C3", "C5_prepack", "C5", "C2", "C4") if k in results]
-    line["all"] = {k: results[k] for k in [k for k in results if k not in last] + last}
+    sys.stderr.write("[bench] all " + json.dumps(results) + "\n")
+    sys.stderr.flush()
     print(json.dumps(line))
     if not parity_ok:
         sys.stderr.write("[bench] PARITY FAILED: " + json.dumps({k: v for k, v in checked.items() if not v["ok"]}) + "\n")
