@@ -194,6 +194,7 @@ namespace {
 int launch_choice(const blkq4::Choice& choice, bool bf16, const blkq4_gemm_args* args) {
   if (choice.family == blkq4::kFamilyDecode) return bf16 ? blkq4_dev_decode_bf16(args) : blkq4_dev_decode(args);
   const bool streaming = choice.family == blkq4::kFamilyStreaming;
+  if (streaming && choice.s.am == blkq4::kRowsPerSlotInLds) return bf16 ? blkq4_dev_staged_bf16(args) : blkq4_dev_staged(args);
   return bf16 ? (streaming ? blkq4_dev_skinny_bf16(args) : blkq4_dev_gemm_bf16(args))
               : (streaming ? blkq4_dev_skinny(args) : blkq4_dev_gemm(args));
 }

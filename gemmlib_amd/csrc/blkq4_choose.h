@@ -285,22 +285,33 @@ inline long streaming_rounds(int row_groups, int col_groups, int neighbours) {
   return (streaming_busiest_xcd(row_groups, col_groups, neighbours) + kComputeUnits / 8 - 1) / (kComputeUnits / 8);
 }
 
+// Rows staged per slice (blkq4_staged.hip): rows of a row group, dealt evenly ...
+inline int staged_rows_per_group(int m, int row_groups) { return (m + row_groups - 1) / row_groups; }
+// ... and the rounds of 64-deep slices that only the older half of eight waves takes, which a SIMD serves first (us with 0,
+// 2 and 4 of them, K = N = 4096: M = 64 6.6, 6.5, 6.5, M = 128 8.9, 8.6, 8.4; M = 16, N = 28672, K = 8192 26.1, 25.9, 26.0;
+// M = 12, N = 4096, K = 11008 11.3, 11.1, 11.3).
+inline int staged_extra_rounds(int waves, int k) { return (waves == 8 && k >= 2048) ? 2 : 0; }
+
 // Launch geometry of one instantiation.  Many more workgroups than the chip holds at once: a workgroup then
 // walks over several column groups (cg, cg + cg_stride, ...) and requests the first slices of the next one
 // while it finishes the current one, so only the first column group of a workgroup waits for its weights with
 // nothing else to do.  The partial tiles then get LDS of their own: the rows stay where they are for the next
 // column group.  (not the sixteen-wave kernel for blocks along N: its walking variant does not fit in 128
 // registers)
+// (Rows staged per slice: one column group per workgroup, however many there are, and a kernel that knows its LDS itself.)
 inline void streaming_geometry(StreamingShape* s, bool row, int n, int k) {
+  if (s->am == kRowsPerSlotInLds) {
+    const int groups = (n / 16 + s->nt - 1) / s->nt, deal = 8 * streaming_neighbours(s->nt, s->waves, s->split);
+    s->cg_stride = (groups + deal - 1) / deal * deal;
+    s->grid = static_cast<uint32_t>(s->cg_stride) * static_cast<uint32_t>(s->row_groups);
+    return;
+  }
   constexpr int kPersistentFactor = 2;  // column groups per workgroup from which on workgroups walk
   // partial tiles of the sum across waves: [wave][tile][row tile][row][16 columns] floats, rows that exist only
   const size_t rows = s->mt == 1 ? (size_t{1} << s->rows_log2) : 16;
   const size_t red_bytes = (s->split == 1) ? 0 : static_cast<size_t>(s->waves) * s->nt * s->mt * rows * 64;
-  const size_t per_slot_bytes = static_cast<size_t>(s->waves) * s->depth * 16 * s->mt * 256;
   // the rows are copied 1 KiB at a time
-  const size_t a_bytes = s->am == kRowsWholeInLds
-                             ? ((((static_cast<size_t>(k) * 2) << s->rows_log2) + 1023) & ~size_t{1023})
-                             : per_slot_bytes;
+  const size_t a_bytes = (((static_cast<size_t>(k) * 2) << s->rows_log2) + 1023) & ~size_t{1023};
   const int group_tiles = s->nt * (s->waves / s->split);
   const int col_groups = (n / 16 + group_tiles - 1) / group_tiles;
   const int per_xcd_round = 8 * streaming_neighbours(s->nt, s->waves, s->split);

@@ -47,8 +47,8 @@ typedef struct {
   int bf16;            /* 1: src and scales are bf16; 0: fp16 */
 } blkq4_prepack_args;
 
-/* Which streaming kernel runs and how it is launched: the template parameters of skinny_mfma_kernel
- * (blkq4_skinny.hip) and the launch geometry derived from them.  Filled in by blkq4::choose() (blkq4_choose.h). */
+/* Which streaming kernel runs and how it is launched: the template parameters of skinny_mfma_kernel (blkq4_skinny.hip,
+ * am = kRowsWholeInLds) or staged_mfma_kernel (blkq4_staged.hip, kRowsPerSlotInLds) and the launch geometry derived from them.  Filled in by blkq4::choose() (blkq4_choose.h). */
 typedef struct {
   int depth, nt, mt, waves, am, split; /* split = waves (the waves split K) or 1 (they do not) */
   int rows_log2, row_groups;
@@ -116,9 +116,11 @@ typedef struct {
 
 int blkq4_dev_prepack(const blkq4_prepack_args* args);
 int blkq4_dev_gemm(const blkq4_gemm_args* args);   /* MFMA tile kernel, every m (made for large m) */
-int blkq4_dev_skinny(const blkq4_gemm_args* args); /* weight-streaming kernel, 1 <= m <= 1024 */
+int blkq4_dev_skinny(const blkq4_gemm_args* args); /* weight-streaming kernel, rows whole in LDS, 1 <= m <= 1024 */
 int blkq4_dev_gemm_bf16(const blkq4_gemm_args* args);   /* the tile kernel with bf16 a, scales, c and bias */
 int blkq4_dev_skinny_bf16(const blkq4_gemm_args* args); /* the same with bf16 a, scales, c and bias */
+int blkq4_dev_staged(const blkq4_gemm_args* args);      /* the streaming kernel with rows staged per slice */
+int blkq4_dev_staged_bf16(const blkq4_gemm_args* args); /* the same with bf16 a, scales, c and bias */
 int blkq4_dev_decode(const blkq4_gemm_args* args);      /* decode kernel: few rows, all of K requested at once, blocks along K */
 int blkq4_dev_decode_bf16(const blkq4_gemm_args* args); /* the same with bf16 a, scales, c and bias */
 int blkq4_dev_gemv_dot(const blkq4_gemm_args* args);    /* fp16 GEMV on the vector ALU (no MFMA): 1 <= m <= 4, blocks along K */

@@ -24,6 +24,10 @@ __device__ __forceinline__ void async_copy_16_once(uint32_t lds_base, const void
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds_base), "v"(offset), "s"(base)
                : "memory", "m0");
 }
+__device__ __forceinline__ void async_copy_4(uint32_t lds_base, const void* base, uint32_t offset) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" ::"s"(lds_base), "v"(offset), "s"(base)
+               : "memory", "m0");
+}
 __device__ __forceinline__ void async_copy_4_flat(uint32_t lds_base, const void* gptr) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_base), "v"(gptr) : "memory", "m0");
 }
@@ -36,6 +40,12 @@ __device__ __forceinline__ uint4 lds_read_16(uint32_t addr, int imm = 0) {
   const auto* p = reinterpret_cast<const __attribute__((address_space(3))) uint8_t*>(addr) + imm;
   const lds_u32x4_t v = *reinterpret_cast<const __attribute__((address_space(3))) lds_u32x4_t*>(p);
   return make_uint4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ uint2 lds_read_8(uint32_t addr, int imm = 0) {
+  typedef uint32_t lds_pair_t __attribute__((ext_vector_type(2)));
+  const auto* p = reinterpret_cast<const __attribute__((address_space(3))) uint8_t*>(addr) + imm;
+  const lds_pair_t v = *reinterpret_cast<const __attribute__((address_space(3))) lds_pair_t*>(p);
+  return make_uint2(v[0], v[1]);
 }
 __device__ __forceinline__ uint32_t lds_read_u16(uint32_t addr, int imm = 0) {
   const auto* p = reinterpret_cast<const __attribute__((address_space(3))) uint8_t*>(addr) + imm;

@@ -1,5 +1,5 @@
-// Weight-streaming kernel for gfx950: decode GEMV, small-batch GEMM and, in row groups of 32, every M
-// for which streaming the weights once per row group beats the tile kernel.
+// Weight-streaming kernel for gfx950, rows whole in LDS: what the decode kernel does not take of the small batches, and, in
+// row groups of 32, a short K.  (Rows staged slice by slice: blkq4_staged.hip.)
 //
 // The work is a stream over the packed weights (K*N/2 bytes plus scales and zero-points) that has to
 // run at HBM speed; everything else is arranged so that the stream is requested as early and as
@@ -14,11 +14,10 @@
 //     multiplied by a zero scale, so the loop has no divergent loads);
 //   - the activation rows are copied into LDS by asynchronous global_load_lds copies, laid out per 32-deep
 //     unit as [unit][row][64 bytes] (16-byte chunks XOR-swizzled with bits 2..3 of the row so that a
-//     fragment read is free of bank conflicts).  When all of K fits, a wave stages the rows of the slices it
-//     will convert itself, once, before its first weight request; otherwise per slot, right before the slot's
-//     weights.  Either way the rows a wave reads are rows it requested itself before the weights it multiplies
-//     them with, requests complete in order, and no barrier is needed: a wave that has its weights has its rows.
-//     (Waves that do not split K share out the copies of all rows and meet at one barrier.)
+//     fragment read is free of bank conflicts).  A wave stages the rows of the slices it will convert itself, once,
+//     before its first weight request: the rows a wave reads are rows it requested itself before the weights it
+//     multiplies them with, requests complete in order, and no barrier is needed: a wave that has its weights has its
+//     rows.  (Waves that do not split K share out the copies of all rows and meet at one barrier.)
 //   - a lane dequantizes its (column, 32 k) of weights once and multiplies them with the matching 32 k of
 //     MT tiles of 16 activation rows through v_mfma_f32_16x16x32_f16 (weights as the row operand: a lane
 //     ends up with 4 consecutive output columns of one activation row per tile);
@@ -101,7 +100,7 @@ constexpr bool kBF = true;
 constexpr bool kBF = false;
 #endif
 
-template <int BS, int NT, int MT, int AM, bool ROW>
+template <int BS, int NT, int MT, bool ROW>
 struct Slot {
   static constexpr int kMeta = (BS == 16) ? 2 : 1;  // quantization blocks inside one 32-deep unit
   uint4 w[NT];
@@ -117,15 +116,14 @@ struct Slot {
 // are summed through LDS) or none (kSplit = 1: every wave has NT column tiles of its own and all of K).
 // DEPTH: k slices (128 deep) a wave keeps in flight.  NT: 16-column tiles per wave that share one activation
 // operand.  MT: 16-row tiles of activations (M <= 16 * MT) that share one conversion of the weights.
-// AM: where the activation rows are (see above).  kRowsWholeInLds: rows_log2 = log2 of the number of rows kept
-// in LDS, a power of two >= M; kRowsPerSlotInLds: kWaves * DEPTH * 16 * MT * 256 bytes of slots.
+// rows_log2 = log2 of the number of rows kept in LDS, a power of two >= M.
 // kRefill: false for one column group (NT * kWaves / kSplit tiles) per workgroup; true for workgroups that walk
 // over the column groups cg, cg + cg_stride, ... (the partial tiles then live at red_offset, behind the rows,
 // which stay) and for waves that do not split K.
 // ROW: quantization blocks run along N (one k, BS columns); S and Z are then in the packed order
 // described in blkq4_device.h and the lane's column group decides which 64 + 32 bytes it fetches per unit.
 // (BF repeats kBF so that the two compilations' kernels carry different names in a trace)
-template <int BS, bool HAS_ZP, int DEPTH, int NT, int MT, int kWaves, int AM, bool ROW, bool kRefill, int kSplit, bool BF = kBF>
+template <int BS, bool HAS_ZP, int DEPTH, int NT, int MT, int kWaves, bool ROW, bool kRefill, int kSplit, bool BF = kBF>
 __global__ __launch_bounds__(64 * kWaves) void skinny_mfma_kernel(const uint16_t* __restrict__ A,
                                                                const uint4* __restrict__ W,
                                                                const uint16_t* __restrict__ S,
@@ -134,10 +132,7 @@ __global__ __launch_bounds__(64 * kWaves) void skinny_mfma_kernel(const uint16_t
                                                                const uint16_t* __restrict__ bias, int M_total, int N,
                                                                int K, int rows_log2, int row_groups,
                                                                int cg_stride, uint32_t red_offset) {
-  constexpr int kMeta = Slot<BS, NT, MT, AM, ROW>::kMeta;
-  constexpr bool A_LDS = AM == kRowsWholeInLds;
-  constexpr int kSlotRows = 16 * MT;                           // kRowsPerSlotInLds: rows staged per slot
-  constexpr int kSlotBytes = kSlotRows * 256;
+  constexpr int kMeta = Slot<BS, NT, MT, ROW>::kMeta;
   // the partial tiles of the sums across waves reuse the LDS of the activation rows (red_offset = 0) or, when
   // the workgroup goes on to another column group and needs the rows again, lie behind them
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
@@ -202,7 +197,7 @@ __global__ __launch_bounds__(64 * kWaves) void skinny_mfma_kernel(const uint16_t
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[t][mt] = float4_t{0.f, 0.f, 0.f, 0.f};
-  Slot<BS, NT, MT, AM, ROW> slot[DEPTH];
+  Slot<BS, NT, MT, ROW> slot[DEPTH];
 
   // Rows to LDS, requested before anything else.  Layout: [pair of 32-deep units][row][128 B], the eight 16-byte
   // chunks of a row's 128 bytes XOR-swizzled with bits 1..3 of the row (the 16 lanes of a fragment read touch 16
@@ -215,12 +210,7 @@ __global__ __launch_bounds__(64 * kWaves) void skinny_mfma_kernel(const uint16_t
   uint32_t a_swz = 0;  // bits 1..3 of the row
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
                             (__attribute__((address_space(3))) uint8_t*)(smem)));
-  if (AM == kRowsPerSlotInLds) {
-    // this wave's slots: DEPTH pieces of [2 pairs][kSlotRows rows][128 B]
-    a_rd = (wave * DEPTH) * kSlotBytes + nl * 128;
-    a_swz = (nl >> 1) & 7;
-  }
-  if (A_LDS) {
+  {
     const int rows = 1 << rows_log2;
     if (kSplit == 1) {
       // every wave needs all of K: the waves share out the copies (copy q fills LDS bytes [1024 q, 1024 q + 1024),
@@ -261,7 +251,7 @@ __global__ __launch_bounds__(64 * kWaves) void skinny_mfma_kernel(const uint16_t
     a_swz = (row >> 1) & 7;
   }
   // unit g of a slice is half g & 1 of pair g >> 1 (a_lane: offset of the pair's row; a_half: which 64 bytes)
-  const uint32_t pair_bytes = (AM == kRowsPerSlotInLds) ? kSlotRows * 128 : (128u << rows_log2);
+  const uint32_t pair_bytes = 128u << rows_log2;
   a_lane[0] = static_cast<uint32_t>(g >> 1) * pair_bytes + a_rd;
   a_lane[1] = static_cast<uint32_t>(g_alt >> 1) * pair_bytes + a_rd;
   const uint32_t a_half[2] = {static_cast<uint32_t>(g & 1) * 4, static_cast<uint32_t>(g_alt & 1) * 4};
@@ -274,20 +264,6 @@ __global__ __launch_bounds__(64 * kWaves) void skinny_mfma_kernel(const uint16_t
   // adds the wave's part to it with 64-bit vector additions: 110 instructions of address arithmetic per slot of four
   // tiles against the 224 of its conversion.)
   const uint32_t m2_lane[2] = {m_lane[0] * 2, m_lane[1] * 2};
-  // rows staged per slot: copy q fills LDS bytes [1024 q, 1024 q + 1024) of the slot, lane l the 16 bytes at 16 l;
-  // a last slice with two units only fetches its first pair twice
-  uint32_t a_copy[(AM == kRowsPerSlotInLds) ? 4 * MT : 1][2];
-  if (AM == kRowsPerSlotInLds) {
-#pragma unroll
-    for (int q = 0; q < 4 * MT; ++q) {
-      const int rr = 8 * q + (lane >> 3);  // (pair, row) index inside the slot
-      const int row = rr % kSlotRows;
-      const int chunk = (lane & 7) ^ ((row >> 1) & 7);
-      const uint32_t in_pair = (static_cast<uint32_t>(min(row, M - 1)) * K + (chunk >> 2) * 32 + (chunk & 3) * 8) * 2;
-      a_copy[q][0] = in_pair + (rr / kSlotRows) * 128;
-      a_copy[q][1] = in_pair;
-    }
-  }
 #define BLKQ4_LOAD_SLOT(dst_, d_, cg_, slice_, keep_, W_, S_, Z_)                                                \
   {                                                                                            \
     const int sl_ = min((slice_), last_slice);                                                 \
@@ -296,13 +272,6 @@ __global__ __launch_bounds__(64 * kWaves) void skinny_mfma_kernel(const uint16_t
     const uint32_t ml_ = alt_ ? m_lane[1] : m_lane[0];                                         \
     const uint32_t ml2_ = alt_ ? m2_lane[1] : m2_lane[0];                                      \
     const uint32_t keep32_ = static_cast<uint32_t>(keep_);                                     \
-    if (AM == kRowsPerSlotInLds) {                                                             \
-      /* requested before the slot's weights, so whoever has the weights has the rows */       \
-      _Pragma("unroll") for (int q = 0; q < 4 * MT; ++q) {                                     \
-        async_copy_16(__builtin_amdgcn_readfirstlane(lds0 + (wave * DEPTH + (d_)) * kSlotBytes + q * 1024), A, \
-                      (alt_ ? a_copy[q][1] : a_copy[q][0]) + static_cast<uint32_t>(sl_) * 256u); \
-      }                                                                                        \
-    }                                                                                          \
     _Pragma("unroll") for (int t = 0; t < NT; ++t) {                                           \
       /* tile t of column group cg_; a tile past the end (last column group only, when the group's */ \
       /* tile count does not divide the number of tiles) re-reads the group's first tile and is    */ \
@@ -347,7 +316,7 @@ __global__ __launch_bounds__(64 * kWaves) void skinny_mfma_kernel(const uint16_t
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) BLKQ4_LOAD_SLOT(slot[d], d, cg, ws + kSplit * d, -1, w0, s0, z0);
   }
-  if constexpr (A_LDS && kSplit == 1) {
+  if constexpr (kSplit == 1) {
     // everything but the requests of the ring just issued has landed: this wave's share of the rows; then
     // everybody's
     constexpr int kLoads = ROW ? NT * (1 + 4 + (HAS_ZP ? 2 : 0)) : NT * (1 + kMeta * (HAS_ZP ? 2 : 1));
@@ -424,41 +393,28 @@ __global__ __launch_bounds__(64 * kWaves) void skinny_mfma_kernel(const uint16_t
   bool own_rows_landed = false;  // wave-uniform
   // converts slot d, which holds local slice li, and multiplies it with the rows
   auto consume = [&](int d, int li) {
-    const Slot<BS, NT, MT, AM, ROW>& cur = slot[d];
+    const Slot<BS, NT, MT, ROW>& cur = slot[d];
     const int slice = ws + kSplit * li;
     const int sl = min(slice, last_slice);
     const uint32_t full = (slice < last_slice || (slice == last_slice && rem == 0)) ? 0xffffffffu : 0u;  // uniform
     const uint32_t okm = full | ((slice == last_slice) ? ok_last : 0u);
       uint4 af[MT][4];  // eight 16-bit activations each
-      // Rows staged by this wave itself were requested before the slot's weights and requests complete in
-      // order: the reads below wait for one of the slot's weight words -- for every slot when the rows are staged
-      // per slot, for the wave's first slot only when it staged the rows of all its slices up front (after that
-      // they are all there, and the reads may run ahead of the weights again).  (Waiting for the copies by count
-      // right behind the first ring's requests instead is slower: C2 4.55 -> 4.73 us.)
+      // Rows staged by this wave itself were requested before its first weights and requests complete in order: the reads
+      // of its first slot wait for one of the slot's weight words (after that all its rows are there, and the reads may run
+      // ahead of the weights again).  (Waiting for the copies by count right behind the first ring's requests instead is
+      // slower: M = 1, K = N = 4096 4.55 -> 4.73 us.)
       uint32_t arrived = 0u;
-      if (AM == kRowsPerSlotInLds) {
-        arrived = zero_once_loaded(cur.w[0].x);
-      } else if (kSplit != 1 && !own_rows_landed) {
+      if (kSplit != 1 && !own_rows_landed) {
         arrived = zero_once_loaded(cur.w[0].x);
         own_rows_landed = true;
       }
-      if (A_LDS) {
+      {
         // (a slot past the wave's last slice holds the last slice's weights with zeroed scales; it is multiplied
         // with rows this wave has staged itself, those of its first slice: 0 times anything finite)
         const int sl_a = (kSplit == 1 || slice <= last_slice) ? sl : ws;
         const bool alt_a = rem != 0 && sl_a == last_slice;
         const uint8_t* ap = a_lds + (static_cast<uint32_t>(4 * sl_a) << (6 + rows_log2)) + (alt_a ? a_lane[1] : a_lane[0]) + arrived;
         const uint32_t half = alt_a ? a_half[1] : a_half[0];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            af[mt][j] = *reinterpret_cast<const uint4*>(ap + mt * 2048 + (((half + j) ^ a_swz) * 16));
-          }
-      } else {
-        // (all four units of a slot hold valid rows, also past the end of K: the lane reads its own unit g)
-        const uint8_t* ap = a_lds + a_lane[0] + d * kSlotBytes + arrived;
-        const uint32_t half = a_half[0];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -597,19 +553,16 @@ hipError_t raise_lds_limit() {
 
 // One kernel instantiation with the launch geometry of the plan (blkq4_choose.h): raises its dynamic-LDS limit,
 // then launches.  What the kernel assumes about the plan is checked here.
-template <int BS, bool HAS_ZP, bool ROW, int DEPTH, int NT, int MT, int kWaves, int AM, int kSplit>
+template <int BS, bool HAS_ZP, bool ROW, int DEPTH, int NT, int MT, int kWaves, int kSplit>
 int launch_kernel(const blkq4_gemm_args* a) {
   const blkq4_streaming_plan& p = a->streaming;
   // partial tiles of the sum across waves, rows that exist only
   const size_t red_rows = MT == 1 ? (size_t{1} << p.rows_log2) : 16;
   const size_t kRedBytes = (kSplit == 1) ? 0 : static_cast<size_t>(kWaves) * NT * MT * red_rows * 64;
-  constexpr size_t kPerSlotBytes = static_cast<size_t>(kWaves) * DEPTH * 16 * MT * 256;
   static_assert(static_cast<size_t>(kWaves) * NT * MT * 16 * 64 <= kMaxLdsBytes, "partial tiles do not fit in LDS");
-  static_assert(AM != kRowsPerSlotInLds || kPerSlotBytes <= kMaxLdsBytes, "slots do not fit in LDS");
   const bool refill = p.refill != 0;
-  if (a->launched_id != nullptr) *a->launched_id = streaming_id(DEPTH, NT, MT, kWaves, AM, kSplit, refill);
-  const size_t a_bytes = AM == kRowsWholeInLds ? ((((static_cast<size_t>(a->k) * 2) << p.rows_log2) + 1023) & ~size_t{1023})
-                                               : kPerSlotBytes;
+  if (a->launched_id != nullptr) *a->launched_id = streaming_id(DEPTH, NT, MT, kWaves, kRowsWholeInLds, kSplit, refill);
+  const size_t a_bytes = (((static_cast<size_t>(a->k) * 2) << p.rows_log2) + 1023) & ~size_t{1023};
   constexpr int kGroupTiles = NT * (kWaves / kSplit);
   constexpr int kXcdRound = 8 * streaming_neighbours(NT, kWaves, kSplit);  // column groups dealt to the XCDs at a time
   const int col_groups = (a->n / 16 + kGroupTiles - 1) / kGroupTiles;
@@ -640,57 +593,46 @@ int launch_kernel(const blkq4_gemm_args* a) {
     if constexpr (ROW && kWaves == 16) {
       return static_cast<int>(hipErrorInvalidValue);
     } else {
-      constexpr auto kernel = skinny_mfma_kernel<BS, HAS_ZP, DEPTH, NT, MT, kWaves, AM, ROW, true, kSplit>;
+      constexpr auto kernel = skinny_mfma_kernel<BS, HAS_ZP, DEPTH, NT, MT, kWaves, ROW, true, kSplit>;
       return launch(kernel, raise_lds_limit<kernel>());
     }
   }
   if constexpr (kSplit == 1) {
     return static_cast<int>(hipErrorInvalidValue);  // waves that do not split K exist in the walking form only
   } else {
-    constexpr auto kernel = skinny_mfma_kernel<BS, HAS_ZP, DEPTH, NT, MT, kWaves, AM, ROW, false, kSplit>;
+    constexpr auto kernel = skinny_mfma_kernel<BS, HAS_ZP, DEPTH, NT, MT, kWaves, ROW, false, kSplit>;
     return launch(kernel, raise_lds_limit<kernel>());
   }
 }
 
-// The shapes that exist, (DEPTH, NT, MT, waves, AM, split): what blkq4::choose() may ask for.  Blocks along N:
+// The shapes that exist, (DEPTH, NT, MT, waves, split): what blkq4::choose() may ask for.  Blocks along N:
 // those with one column tile per wave (28 registers of packed weights, scales and zero-points per slot and tile).
-#define BLKQ4_W kRowsWholeInLds
-#define BLKQ4_P kRowsPerSlotInLds
 #define BLKQ4_STREAMING_SHAPES(X)                                                                          \
   /* row groups of 32 */                                                                                   \
-  X(2, 1, 2, 8, BLKQ4_W, 8) X(2, 2, 2, 8, BLKQ4_W, 8) X(2, 4, 2, 8, BLKQ4_W, 8) X(2, 6, 2, 8, BLKQ4_W, 8)  \
-  X(2, 8, 2, 8, BLKQ4_W, 8)                                                                                \
-  X(2, 1, 2, 8, BLKQ4_P, 8) X(2, 2, 2, 8, BLKQ4_P, 8) X(2, 4, 2, 8, BLKQ4_P, 8) X(2, 6, 2, 8, BLKQ4_P, 8)  \
-  X(2, 8, 2, 8, BLKQ4_P, 8)                                                                                \
+  X(2, 1, 2, 8, 8) X(2, 2, 2, 8, 8) X(2, 4, 2, 8, 8) X(2, 6, 2, 8, 8) X(2, 8, 2, 8, 8)                     \
   /* waves with column tiles of their own */                                                               \
-  X(4, 1, 1, 4, BLKQ4_W, 1)                                                                                \
-  /* wide layers, rows staged per slice */                                                                 \
-  X(2, 4, 1, 4, BLKQ4_P, 4) X(2, 4, 1, 8, BLKQ4_P, 8)                                                      \
-  X(2, 5, 1, 4, BLKQ4_P, 4) X(2, 6, 1, 4, BLKQ4_P, 4) X(2, 7, 1, 4, BLKQ4_P, 4)                            \
-  X(2, 5, 1, 8, BLKQ4_P, 8) X(2, 6, 1, 8, BLKQ4_P, 8) X(2, 7, 1, 8, BLKQ4_P, 8)                            \
+  X(4, 1, 1, 4, 1)                                                                                         \
   /* up to 16 rows, the waves split K */                                                                   \
-  X(4, 1, 1, 8, BLKQ4_W, 8) X(4, 2, 1, 8, BLKQ4_W, 8) X(4, 3, 1, 8, BLKQ4_W, 8) X(2, 1, 1, 8, BLKQ4_W, 8)  \
-  X(2, 1, 1, 16, BLKQ4_W, 16) X(2, 2, 1, 16, BLKQ4_W, 16) X(2, 3, 1, 16, BLKQ4_W, 16)                      \
-  X(4, 1, 1, 8, BLKQ4_P, 8) X(4, 2, 1, 8, BLKQ4_P, 8) X(4, 3, 1, 8, BLKQ4_P, 8)                            \
-  X(8, 1, 1, 4, BLKQ4_W, 4) X(4, 1, 1, 4, BLKQ4_W, 4) X(4, 2, 1, 4, BLKQ4_W, 4) X(4, 3, 1, 4, BLKQ4_W, 4)
+  X(4, 1, 1, 8, 8) X(4, 2, 1, 8, 8) X(4, 3, 1, 8, 8) X(2, 1, 1, 8, 8)                                      \
+  X(2, 1, 1, 16, 16) X(2, 2, 1, 16, 16) X(2, 3, 1, 16, 16)                                                 \
+  X(8, 1, 1, 4, 4) X(4, 1, 1, 4, 4) X(4, 2, 1, 4, 4) X(4, 3, 1, 4, 4)
 
 template <int BS, bool HAS_ZP, bool ROW>
 int launch_plan(const blkq4_gemm_args* a) {
   const blkq4_streaming_plan& p = a->streaming;
-#define BLKQ4_TRY(D_, NT_, MT_, W_, AM_, S_)                                                               \
-  if (p.depth == D_ && p.nt == NT_ && p.mt == MT_ && p.waves == W_ && p.am == AM_ && p.split == S_) {      \
+  if (p.am != kRowsWholeInLds) return static_cast<int>(hipErrorInvalidValue);
+#define BLKQ4_TRY(D_, NT_, MT_, W_, S_)                                                                    \
+  if (p.depth == D_ && p.nt == NT_ && p.mt == MT_ && p.waves == W_ && p.split == S_) {                     \
     if constexpr (ROW && NT_ > 1) {                                                                        \
       return static_cast<int>(hipErrorInvalidValue);                                                       \
     } else {                                                                                               \
-      return launch_kernel<BS, HAS_ZP, ROW, D_, NT_, MT_, W_, AM_, S_>(a);                                 \
+      return launch_kernel<BS, HAS_ZP, ROW, D_, NT_, MT_, W_, S_>(a);                                      \
     }                                                                                                      \
   }
   BLKQ4_STREAMING_SHAPES(BLKQ4_TRY)
 #undef BLKQ4_TRY
   return static_cast<int>(hipErrorInvalidValue);  // a shape that does not exist
 }
-#undef BLKQ4_W
-#undef BLKQ4_P
 
 template <int BS>
 int launch_skinny(const blkq4_gemm_args* a) {
