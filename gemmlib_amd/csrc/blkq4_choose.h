@@ -338,6 +338,23 @@ inline void streaming_geometry(StreamingShape* s, bool row, int n, int k) {
   s->refill = (cg_stride < col_groups || s->split == 1) ? 1 : 0;
 }
 
+// What the cost of a workgroup depends on besides its shape (the tile kernel's factors are below).
+enum TileCostRow { kCostPlain = 0, kCostBf16 = 1, kCostBlocksAlongN = 2, kCostBlocksOf16 = 4 };  // bits
+inline int tile_cost_row(bool column_wise, bool bf16, int block_size) {
+  return (bf16 ? kCostBf16 : 0) | (!column_wise ? kCostBlocksAlongN : 0) | (block_size == 16 ? kCostBlocksOf16 : 0);
+}
+
+// Rows staged per slice, more than 16 of them: rounds of workgroups as the busiest XCD has them, a workgroup's time growing
+// with its column tiles and K.  Least squares over 527 measured (shape, column tiles) pairs, blocks along K, M = 40 ... 512,
+// N = 4096 ... 28672, K = 1024 ... 13824, fp16 and bf16, every block size, plans up to a third behind the shape's best one:
+// 6.7 % rms, within 23 %.  (Blocks of 16, and bf16, cost the same twelfth more each.)
+inline double staged_estimate_us(int row_groups, int n, int k, int nt, int cost_row) {
+  const long rounds = streaming_rounds(row_groups, (n / 16 + nt - 1) / nt, streaming_neighbours(nt, 8, 8));
+  const double kk = static_cast<double>(k) / 1024.0;
+  const double per_tile = 0.36 + ((cost_row & kCostBlocksOf16) ? 0.043 : 0.0) + ((cost_row & kCostBf16) ? 0.043 : 0.0);
+  return 1.5 + static_cast<double>(rounds) * (1.56 + kk * (0.23 + nt * per_tile));
+}
+
 inline StreamingShape streaming_shape(bool row, int m, int n, int k, int block_size = 64) {
   StreamingShape s{};
   auto set = [&](int depth, int nt, int mt, int waves, int am, int split) {
@@ -345,36 +362,24 @@ inline StreamingShape streaming_shape(bool row, int m, int n, int k, int block_s
   };
   s.row_groups = 1;
   if (m > 16) {
-    // Row groups of 32 rows (two row tiles share one conversion of the weights), eight waves.  A workgroup's time
-    // grows with its column tiles -- measured at K = 4096: 3.0 + 1.73 us per tile (M = 128, N = 4096 with 4, 6 and 8
-    // tiles: 11.6, 15.2, 18.5 us) -- and an XCD with more workgroups than compute units takes longer than their number
-    // says: 1.45 x workgroups per unit x one workgroup's time, at least the busiest unit's whole number of them
-    // (M = 96, K = N = 4096: 3 per unit of one tile, 4.7 us each by that line, take 19.9 us, 1.5 per unit of two tiles,
-    // 6.5 us each, 14.5; N = 5152: 1.97 per unit of two tiles 20.1).  As many tiles per workgroup (1, 2, 4, 6, 8) as make
-    // that smallest (M = 64, N = 11008: 344 workgroups of four tiles 21.8 us, 230 of six 15.9; M = 96, N = 5152: two tiles
-    // 20.1, six 15.5).  Blocks along N: 28 registers of packed weights, scales and zero-points per slot and tile, so one
-    // tile.
+    // Row groups of up to 32 rows (one conversion of the weights serves them all), eight waves, rows staged per slice: whole
+    // rows in LDS, which a short K allows, are slower (M = 80 ... 128, N = 4096, K = 1024 7.0 against 4.8 us; blocks along N,
+    // M = 24, N = 4096, K = 1024 4.9 against 3.9).  As many column tiles per workgroup (1, 2, 4, 6, 8) as the estimate likes
+    // best.  Blocks along N: one.
     s.row_groups = (m + 31) / 32;
     s.rows_log2 = 5;
     int nt = 1;
     if (!row) {
       double best = 0.0;
       for (const int t : {1, 2, 4, 6, 8}) {
-        const double per_unit = static_cast<double>(streaming_busiest_xcd(s.row_groups, (n / 16 + t - 1) / t, streaming_neighbours(t, 8, 8))) /
-                                (kComputeUnits / 8);
-        const double whole = static_cast<double>(static_cast<long>(per_unit + 0.999));  // the busiest unit's workgroups
-        const double cost = (per_unit <= 1.0 ? 1.0 : (1.45 * per_unit > whole ? 1.45 * per_unit : whole)) * (3.0 + 1.73 * t);
-        if (t == 1 || cost < best) {
-          best = cost;
+        const double us = staged_estimate_us(s.row_groups, n, k, t, block_size == 16 ? kCostBlocksOf16 : kCostPlain);
+        if (t == 1 || us < best) {
+          best = us;
           nt = t;
         }
       }
     }
-    // the rows whole in LDS only while they are a small part of it: at K = 2048 (128 KB) staging them slice by slice is
-    // a tenth faster (M = 80 ... 128, N = 4096: 7.4 - 7.6 against 8.2 - 8.3 us), at K = 1024 they are level
-    // (blocks along K; with blocks along N whole rows stay ahead, M = 24 ... 96, K = 2048: 8.1 - 11.6 against 9.8 - 15.7 us)
-    const bool rows_fit = static_cast<size_t>(k) * 2 * 32 <= kMaxLdsBytes && (row || k <= 1536);
-    set(2, nt, 2, 8, rows_fit ? kRowsWholeInLds : kRowsPerSlotInLds, 8);
+    set(2, nt, 2, 8, (row && k <= 2560) ? kRowsWholeInLds : kRowsPerSlotInLds, 8);
     streaming_geometry(&s, row, n, k);
     return s;
   }
@@ -601,10 +606,6 @@ struct TileCost {
 // 5 % behind the best one for 4 of the 50, 3 of the 36 and 3 of the 36 shapes (up to 30 %: 128 x 128 tiles on half the
 // chip where a split or a larger tile wins) and, with bf16's factors alone, for 7 and 3 of the 24 + 24 shapes of the
 // combinations; with the factors as they are here for 1, 1, 0, 0 and 0.
-enum TileCostRow { kCostPlain = 0, kCostBf16 = 1, kCostBlocksAlongN = 2, kCostBlocksOf16 = 4 };  // bits
-inline int tile_cost_row(bool column_wise, bool bf16, int block_size) {
-  return (bf16 ? kCostBf16 : 0) | (!column_wise ? kCostBlocksAlongN : 0) | (block_size == 16 ? kCostBlocksOf16 : 0);
-}
 inline TileCost tile_cost(const TileShape& t, int row = kCostPlain) {
   // 64 x 128, 128 x 128, 128 x 256, 256 x 256, 160 x 256, 192 x 256
   static constexpr TileCost kPlain[6] = {{0.29, 0.00065, 1.0, 192}, {0.32, 0.0015, 2.0, 128}, {0.65, 0.0019, 2.0, 128},
@@ -819,19 +820,22 @@ inline TileShape tile_plan(bool column_wise, int m, int n, int k, size_t workspa
 // it has more workgroups than compute units, with whole rounds of them.
 constexpr uint64_t kStreamingMaxWeights = uint64_t{1} << 33;
 
-inline bool streaming_kernel_takes(bool column_wise, int m, int n, int k, const StreamingShape& s, double tile_us, int row = kCostPlain) {
+inline bool streaming_kernel_takes(bool column_wise, int m, int n, int k, const StreamingShape& s, double tile_us, bool tile_split, int row = kCostPlain) {
   // its offsets into the packed weights (K N / 2 bytes) are 32 bits wide (so are the other kernels': the entry points
   // refuse such problems before any kernel is chosen)
   if (static_cast<uint64_t>(k) * static_cast<uint64_t>(n) >= kStreamingMaxWeights) return false;
   if (m <= 16) return true;
   if (m > kStreamingMaxRows) return false;
   const long row_groups = s.row_groups;
+  // Blocks along K against tiles without a split: by the estimate of rows staged per slice, which has to promise a tenth
+  // less (both estimates are off by 7 % rms).  Of 190 measured shapes, M = 40 ... 512, this hands it eight more than the
+  // lines below do, each 10 - 34 % faster (M = 160, N = 4096, K = 3072 13.0 -> 9.5 us, M = 128, K = 1024 7.3 -> 4.8, M = 64,
+  // N = 14336 19.7 -> 17.4); what it would win by less stays in tiles (M = 200 ... 256, N = 4096: 4 - 15 %).
+  if (column_wise && !tile_split && 1.1 * staged_estimate_us(s.row_groups, n, k, s.nt, row) < tile_us) return true;
   const long streaming_groups = row_groups * ceil_div(n / 16, s.nt);
   // (row groups of 32: the waves split K, a column group is s.nt tiles)
   const long col_groups = ceil_div(n / 16, s.nt);
-  const long rounds = s.cg_stride >= col_groups
-                          ? streaming_rounds(s.row_groups, static_cast<int>(col_groups), streaming_neighbours(s.nt, s.waves, s.split))
-                          : ceil_div(streaming_groups, kComputeUnits);
+  const long rounds = streaming_rounds(s.row_groups, static_cast<int>(col_groups), streaming_neighbours(s.nt, s.waves, s.split));
   if (column_wise && (m <= 64 || k < 4096)) {
     // (More row groups with a short K too: the product further down has no fixed part and said 5.6 us for M = 256,
     // K = 1024, N = 4096, which takes 11.3 -- and the 128 x 32 tiles whose waves split the k tile 6.7; this line says 12.1.
@@ -888,7 +892,7 @@ inline Choice choose(bool column_wise, bool bf16, int m, int n, int k, size_t wo
   const int row = tile_cost_row(column_wise, bf16, block_size);
   c.t = tile_plan(column_wise, m, n, k, workspace_capacity, row);
   const double tile_us = (column_wise && m <= 64) ? few_rows_tile_estimate_us(c.t, k, m > 32 ? row : kCostPlain) : tile_estimate_us(c.t, k, row);
-  c.family = streaming_kernel_takes(column_wise, m, n, k, c.s, tile_us, row) ? kFamilyStreaming : kFamilyTile;
+  c.family = streaming_kernel_takes(column_wise, m, n, k, c.s, tile_us, c.t.split_k > 1, row) ? kFamilyStreaming : kFamilyTile;
   return c;
 }
 
