@@ -728,13 +728,14 @@ __global__ __launch_bounds__(64 * (WM * WN * KW + PW))
   if (SK && parts > 1) {
     // Partial tile of (split tile st, part): [wave][row tile][fragment][g][half][lane] pairs of floats -- a
     // wave's store or load instruction covers 512 consecutive bytes.  The partial tiles and the counters are
-    // exchanged between workgroups on different XCDs, whose L2 caches do not see each other's lines.  So, per
-    // workgroup and not per wave (the cache operations act on the XCD's whole L2, and every invalidate throws
-    // away the operands the other workgroups of the XCD are working on): once all waves' stores have completed,
-    // ONE thread writes the L2's dirty lines back (release) and counts the workgroup in; in the workgroup that
-    // arrives last, ONE thread invalidates (acquire) before anybody reads the other parts.  The accesses
-    // themselves are device-scope atomic accesses, which bypass the compute unit's own cache.  (A workspace in
-    // uncached memory needs none of the cache operations; measured, that saves 1 us of 18 and is not used.)
+    // exchanged between workgroups on different XCDs, whose L2 caches do not see each other's lines, by device-scope
+    // atomic accesses: they bypass the compute unit's cache, a store is written through L2 and acknowledged when it is
+    // visible to the device.  So a wave that has waited for its stores has released them, and ONE thread per workgroup
+    // counts the workgroup in behind a barrier.  (A release fence there would also write back the XCD's whole L2, which
+    // holds nothing of this exchange: the workgroups of an XCD queue up for it.  128 x 128 tiles, fp16, blocks of 64, with the
+    // fence and without: M = 256, N = K = 4096 in 3 parts 19.1 and 18.1 us, K = 11008 in 4 parts 32.9 and 31.5, M = 128,
+    // N = 11008, K = 4096 in 2 parts 22.1 and 21.4.)  In the workgroup that arrives last, one thread invalidates
+    // (acquire, 0.2 us) before anybody reads the other parts.
     constexpr int kTilePairs = kComputeWaves * RT * NT * 8 * 64;  // 8-byte pairs per partial tile
     constexpr uint32_t kFlagOffset = kStages * St::kBytes - 64;   // behind the epilogue's staging area
     const int st = tile - whole_tiles;
@@ -753,10 +754,9 @@ __global__ __launch_bounds__(64 * (WM * WN * KW + PW))
           const uint64_t v = static_cast<uint64_t>(__float_as_uint(lo)) | static_cast<uint64_t>(__float_as_uint(hi)) << 32;
           __hip_atomic_store(mine + ((r * NT + t) * 8 + g2) * 64, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-    wait_vmcnt<0>();  // this wave's stores have completed
+    wait_vmcnt<0>();  // this wave's stores have been acknowledged
     block_barrier();  // every wave's have
     if (tid == 0) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
       const int arrived = __hip_atomic_fetch_add(&counters[st], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (arrived == parts - 1) {
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
