@@ -195,6 +195,9 @@ int launch_choice(const blkq4::Choice& choice, bool bf16, const blkq4_gemm_args*
   if (choice.family == blkq4::kFamilyDecode) return bf16 ? blkq4_dev_decode_bf16(args) : blkq4_dev_decode(args);
   const bool streaming = choice.family == blkq4::kFamilyStreaming;
   if (streaming && choice.s.am == blkq4::kRowsPerSlotInLds) return bf16 ? blkq4_dev_staged_bf16(args) : blkq4_dev_staged(args);
+  if (!streaming && blkq4::tile_dealt_k_tiles(choice.t, args->k, args->column_wise != 0, bf16, args->block_size, args->zero_points != nullptr)) {
+    return bf16 ? blkq4_dev_kdeal_bf16(args) : blkq4_dev_kdeal(args);
+  }
   return bf16 ? (streaming ? blkq4_dev_skinny_bf16(args) : blkq4_dev_gemm_bf16(args))
               : (streaming ? blkq4_dev_skinny(args) : blkq4_dev_gemm(args));
 }

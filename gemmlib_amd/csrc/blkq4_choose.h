@@ -67,6 +67,22 @@ inline uint64_t decode_id(bool row, int rows, int nt, int waves, int depth) {
   return 4ull << 60 | static_cast<uint64_t>(row ? 1 : 0) << 32 | static_cast<uint64_t>(rows) << 24 | static_cast<uint64_t>(nt) << 16 |
          static_cast<uint64_t>(waves) << 8 | static_cast<uint64_t>(depth);
 }
+// 64 x 128 tiles run one of two kernels: waves with columns of their own (blkq4_gemm.hip), or waves that are dealt whole k
+// tiles (blkq4_kdeal.hip), which take a quarter to a third less per k tile and 1.1 us more in all (their first round is four
+// k tiles, and they sum four tiles of accumulators at the end).  So by the k tiles of a workgroup; fp16, M = 256, N = 4096,
+// unsplit, columns of their own against dealt k tiles:
+//   blocks of 64 along K            K = 1024  7.9 and 8.6 us, 2048 11.3 and 11.2, 2560 13.5 and 12.7, 4096 18.8 and 17.3
+//                                   (M = 512: 9.3 and 10.0, 14.1 and 14.5, 16.7 and 16.5, 25.0 and 22.5)
+//   along N without zero-points     7.3 and 8.3, 11.0 and 11.0, 13.0 and 12.5, 18.8 and 16.9
+//   blocks of 16                    8.5 and 8.4, 12.8 and 12.1 (K = 1536 10.7 and 10.3), 15.3 and 13.7, 21.7 and 19.0
+//   bf16, blocks of 32              9.2 and 9.1, 14.1 and 12.6 (K = 1536 11.5 and 10.8), 16.8 and 14.6, 24.5 and 19.9
+//   along N with zero-points        8.5 and 9.0, 13.2 and 12.7 (K = 1536 10.9 and 10.8), 15.8 and 14.5, 22.9 and 20.2
+inline bool tile_dealt_k_tiles(const TileShape& t, int k, bool column_wise, bool bf16, int block_size, bool has_zp) {
+  if (t.kw == 4 && t.rt == 2 && t.nt == 4) return true;  // asked for by name
+  if (!(t.kw == 1 && t.rt == 2 && t.nt == 1 && t.wm == 1 && t.wn == 4 && t.pw == 4)) return false;
+  const int k_tiles = k / 64 / (t.split_k > 1 ? t.split_k : 1);
+  return k_tiles >= ((bf16 || block_size == 16) ? 24 : (!column_wise && has_zp) ? 32 : 40);
+}
 inline uint64_t choice_id(const Choice& c) {
   if (c.family == kFamilyDecode) return decode_id(c.d.row != 0, c.d.rows, c.d.nt, c.d.waves, c.d.depth);
   return c.family == kFamilyStreaming

@@ -61,7 +61,7 @@ typedef struct {
 
 /* Which tile kernel runs: wm x wn computing waves of (32 rt) x (32 nt) outputs, pw producer waves.
  * kw = 4 (with wm = wn = 1): four computing waves share the one (32 rt) x (32 nt) tile and split every 64-deep k tile
- * between them; kw = 1 otherwise.
+ * between them, or (rt = 2, nt = 4, blkq4_kdeal.hip) take the k tiles in turn; kw = 1 otherwise.
  * split_k > 1: the last split_tiles tiles of the tile order are computed by split_k workgroups each, which
  * leave fp32 partial tiles in the workspace; the last of them to finish sums them in a fixed order.
  * xcd_rows: 0, or into how many row bands (1, 2, 4 or 8) a round of 256 tiles is cut for the 8 XCDs, each of which then
@@ -119,6 +119,8 @@ int blkq4_dev_gemm(const blkq4_gemm_args* args);   /* MFMA tile kernel, every m 
 int blkq4_dev_skinny(const blkq4_gemm_args* args); /* weight-streaming kernel, rows whole in LDS, 1 <= m <= 1024 */
 int blkq4_dev_gemm_bf16(const blkq4_gemm_args* args);   /* the tile kernel with bf16 a, scales, c and bias */
 int blkq4_dev_skinny_bf16(const blkq4_gemm_args* args); /* the same with bf16 a, scales, c and bias */
+int blkq4_dev_kdeal(const blkq4_gemm_args* args);       /* the 64 x 128 tiles, waves dealt whole k tiles */
+int blkq4_dev_kdeal_bf16(const blkq4_gemm_args* args);  /* the same with bf16 a, scales, c and bias */
 int blkq4_dev_staged(const blkq4_gemm_args* args);      /* the streaming kernel with rows staged per slice */
 int blkq4_dev_staged_bf16(const blkq4_gemm_args* args); /* the same with bf16 a, scales, c and bias */
 int blkq4_dev_decode(const blkq4_gemm_args* args);      /* decode kernel: few rows, all of K requested at once, blocks along K */

@@ -62,6 +62,10 @@ __device__ __forceinline__ void lds_write_16(uint32_t addr, int imm, uint32_t x,
   auto* p = reinterpret_cast<__attribute__((address_space(3))) uint8_t*>(addr) + imm;
   *reinterpret_cast<__attribute__((address_space(3))) lds_u32x4_t*>(p) = lds_u32x4_t{x, y, z, w};
 }
+__device__ __forceinline__ void lds_write_4(uint32_t addr, int imm, uint32_t v) {
+  auto* p = reinterpret_cast<__attribute__((address_space(3))) uint8_t*>(addr) + imm;
+  *reinterpret_cast<__attribute__((address_space(3))) uint32_t*>(p) = v;
+}
 typedef uint32_t lds_u32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void lds_write_8(uint32_t addr, int imm, uint32_t lo, uint32_t hi) {
   auto* p = reinterpret_cast<__attribute__((address_space(3))) uint8_t*>(addr) + imm;

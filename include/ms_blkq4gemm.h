@@ -273,8 +273,8 @@ int blkq4_gemm_plan_sm80(
  * cost model.  `plan` is text:
  *   "auto"                                     what the cost model picks (then identical to the entry points above);
  *   "tile RT NT WM WN PW KW PARTS [BANDS]"     the tile kernel: WM x WN computing waves of (32 RT) x (32 NT) outputs, PW
- *                                              producer waves, KW = 4 for the tiles whose waves split the k tile (else
- *                                              1), the tiles of the last round shared out over PARTS workgroups along K;
+ *                                              producer waves, KW = 4 for the tiles whose waves split the k tile or
+ *                                              (2 4 1 1 4 4) take whole k tiles in turn (else 1), the tiles of the last round shared out over PARTS workgroups along K;
  *                                              BANDS (optional; 1, 2, 4 or 8): every whole round of 256 tiles is dealt to
  *                                              the 8 XCDs in blocks, BANDS row bands x 8 / BANDS column bands; 0 or
  *                                              absent: every eighth tile of the column-major order per XCD;

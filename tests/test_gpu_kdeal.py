@@ -1,0 +1,56 @@
+"""The 64 x 128 tiles whose waves are dealt whole k tiles (blkq4_kdeal.hip), asked for by name: the reference's exact
+construction (test/blkq4_fp16_gemm_sm80_test.cu:194-256,469-472) comes out bit for bit where the kernel can go wrong --
+fewer k tiles than waves, rounds that not every wave has, more and fewer rounds than the ring is long, parts of unequal
+length, rows and columns that end inside a tile, column groups past the last one."""
+
+import pytest
+import torch
+
+from test_gpu_gemm import bits_of, check_plans_exact, exact_problem
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # block size, zero-points, rows, columns, K: 1, 2, 4 and 5 k tiles
+    (64, True, 1, 64, 64), (32, False, 63, 192, 128), (16, True, 64, 128, 256), (64, False, 65, 320, 320),
+    # 8, 11, 12, 9, 16 and 33 k tiles: two to nine rounds of four
+    (32, True, 100, 128, 512), (16, False, 130, 448, 704), (16, True, 7, 1088, 768), (64, True, 129, 576, 576),
+    (32, True, 64, 64, 1024), (16, True, 193, 192, 2112),
+]
+
+
+@pytest.mark.parametrize("bs,has_offsets,m,n,k", CASES)
+@pytest.mark.parametrize("column_wise", [True, False])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_every_form_is_exact(oracle, capi, device, bs, has_offsets, m, n, k, column_wise, bf16):
+    plans = [f"tile 2 4 1 1 4 4 {parts}" for parts in (1, 2, 3) if parts <= k // 64]
+    check_plans_exact(oracle, capi, device, bs, has_offsets, column_wise, m, n, k, plans, bf16)
+
+
+@pytest.mark.parametrize("bs,n", [(16, 96), (32, 32), (32, 416)])
+@pytest.mark.parametrize("column_wise", [True, False])
+def test_columns_that_end_inside_a_pair_of_fragments(oracle, capi, device, bs, n, column_wise):
+    check_plans_exact(oracle, capi, device, bs, True, column_wise, 66, n, 448, ["tile 2 4 1 1 4 4 1", "tile 2 4 1 1 4 4 2"], False)
+
+
+@pytest.mark.parametrize("bs,has_offsets,column_wise,m,n,k,bf16", [
+    (64, True, True, 500, 4096, 2624, False), (16, False, True, 500, 4096, 1600, False), (32, True, False, 150, 4096, 4096, False),
+    (64, True, False, 160, 8192, 2048, True)])
+def test_as_the_library_chooses_it_with_a_bias_and_the_same_bits_every_time(oracle, capi, device, bs, has_offsets, column_wise, m, n,
+                                                                            k, bf16):
+    assert capi.gemm_plan(bs, column_wise, m, n, k, has_offsets, bf16)[2].startswith("tile: 64 x 128, 4 + 4 waves")
+    a, q_w, q_s, q_zp, _ = exact_problem(oracle, capi, device, bs, has_offsets, column_wise, m, n, k, bf16)
+    a = torch.randn(m, k, generator=torch.Generator().manual_seed(k)).to(a.dtype).to(device)
+    bias = (torch.randn(n, generator=torch.Generator().manual_seed(n)) * 0.5).to(a.dtype).to(device)
+    first = None
+    for _ in range(3):
+        out, with_bias, general = (torch.full((m, n), float("nan"), dtype=a.dtype, device=device) for _ in range(3))
+        capi.gemm(bs, column_wise, m, n, k, a, q_w, q_s, q_zp, out, bf16=bf16)
+        capi.gemm(bs, column_wise, m, n, k, a, q_w, q_s, q_zp, with_bias, bias=bias, bf16=bf16)
+        capi.gemm_with_plan("tile 4 1 1 4 4 1 1", bs, column_wise, m, n, k, a, q_w, q_s, q_zp, general, bf16=bf16)
+        torch.cuda.synchronize()
+        first = bits_of(out) if first is None else first
+        assert (bits_of(out) == first).all()   # the waves' sums, and the parts, are added in a fixed order
+        assert (bits_of(with_bias) == bits_of(out + bias)).all()
+        # the same 32-bit sums in another order: of outputs rounded to 11 (8) bits some are rounded the other way
+        assert (out.double() - general.double()).norm() <= (2 ** -8 if bf16 else 2 ** -11) * general.double().norm()
