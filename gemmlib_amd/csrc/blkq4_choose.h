@@ -24,7 +24,7 @@ constexpr int kStreamingMaxRows = 1024;
 
 // Where the streaming kernel's waves find their activation fragments.
 constexpr int kRowsWholeInLds = 1;    // all rows, all of K, staged once per workgroup
-constexpr int kRowsPerSlotInLds = 2;  // 16 * MT rows x 128 k staged per slot, private to the wave
+constexpr int kRowsPerSlotInLds = 2;  // 16 * MT rows x 64 k staged per slice, private to the wave
 
 constexpr int kFamilyStreaming = 0;  // weight-streaming kernel (blkq4_skinny.hip)
 constexpr int kFamilyTile = 1;       // MFMA tile kernel (blkq4_gemm.hip)

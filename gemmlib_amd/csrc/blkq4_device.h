@@ -48,7 +48,8 @@ typedef struct {
 } blkq4_prepack_args;
 
 /* Which streaming kernel runs and how it is launched: the template parameters of skinny_mfma_kernel (blkq4_skinny.hip,
- * am = kRowsWholeInLds) or staged_mfma_kernel (blkq4_staged.hip, kRowsPerSlotInLds) and the launch geometry derived from them.  Filled in by blkq4::choose() (blkq4_choose.h). */
+ * am = kRowsWholeInLds) or staged_mfma_kernel (blkq4_staged.hip, kRowsPerSlotInLds) and the launch geometry derived from
+ * them.  Filled in by blkq4::choose() (blkq4_choose.h). */
 typedef struct {
   int depth, nt, mt, waves, am, split; /* split = waves (the waves split K) or 1 (they do not) */
   int rows_log2, row_groups;
