@@ -95,21 +95,21 @@ COUNTER_KIB = {  # name: (FETCH_SIZE, WRITE_SIZE)
     "C5_prepack": (229410.8, 157706.9),
     "C4r": (34415.1, 16386.6),
     "C2r": (4428.1, 8.0),
-    "C1": (869.0, 128.0),
-    "M128": (8649.1, 1024.0),
-    "M256": (14387.1, 2048.0),
-    "M512": (17233.5, 4183.2),
+    "C1": (872.6, 128.0),
+    "M128": (8758.1, 1024.0),
+    "M256": (14388.5, 2048.0),
+    "M512": (17221.1, 4096.0),
     "M768N11K": (60863.0, 16513.7),
-    "M256K11K": (43374.1, 19434.3),
+    "M256K11K": (43372.6, 19431.3),
     "V128K": (136348.8, 250.8),
-    "B16": (64097.7, 896.0),
+    "B16": (67139.8, 896.0),
     "C4b": (34440.5, 16387.2),
     "C2b": (4418.6, 8.0),
 }
 
 
 TRAFFIC_KERNEL = {  # what blkq4_gemm_plan_sm80 said the workload runs when its counters were taken
-    "C1": "streaming: 8 waves splitting K, 1 column tile(s) x 32 rows, 2 slices in flight, rows whole in LDS, 2 row group(s), 128 workgroups",
+    "C1": "streaming: 8 waves splitting K, 1 column tile(s) x 32 rows, 2 slices in flight, rows staged per slice, 2 row group(s), 128 workgroups",
     "C2": "decode: 8 waves splitting K, 4 slices requested by each, 1 column tile(s) x 1 row(s), 256 workgroups",
     "C3": "decode: 8 waves splitting K, 4 slices requested by each, 3 column tile(s) x 16 row(s), 230 workgroups",
     "C4": "tile: 128 x 256, 4 + 4 waves, 256 tiles, blocks of 4 x 8 tiles per XCD",

@@ -24,9 +24,12 @@
 // a kernel that only copies, for 48 rows on 11008 x 4096, takes 5.4 us for the rows, 5.8 for the weights and 9.1 at best for
 // both, whatever the number of waves, the depth and the order of the requests -- and beside that the vector instructions of
 // the conversion share their issue port with the MFMAs, at 1.6 (M = 512) to 2.0 GHz (M = 48): the chip is power limited.
-// fp16, blocks of 64, K = 4096, us, against the kernel before (128-deep slices, weights in registers, refilled after use):
+// fp16, blocks of 64, K = 4096, us, against the kernel before (128-deep slices, weights in registers, refilled after use), a few
+// weight sets in turn that the Infinity Cache holds:
 //   M = 64, N = 4096 8.4 -> 6.5; M = 128, N = 4096 11.4 -> 8.6; M = 48, N = 11008 15.9 -> 13.2; M = 32, N = 11008 12.7 ->
 //   11.1; M = 12, N = 128256 58.7 -> 55.8; M = 12, N = 4096, K = 11008 11.8 -> 11.0; M = 16, N = 28672, K = 8192 27.9 -> 25.9.
+// From HBM (600 MB of weight sets in turn): M = 64, N = 4096 8.3 -> 8.2; M = 128, N = 4096 11.3 -> 10.4; M = 48, N = 11008
+//   15.9 -> 13.7; M = 16, N = 28672, K = 8192 27.3 -> 26.2.
 
 #include <hip/hip_runtime.h>
 
