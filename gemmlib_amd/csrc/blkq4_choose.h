@@ -287,6 +287,21 @@ inline int staged_rows_per_group(int m, int row_groups) { return (m + row_groups
 // M = 12, N = 4096, K = 11008 11.3, 11.1, 11.3).
 constexpr int staged_extra_rounds(int waves, int k) { return (waves == 8 && k >= 2048) ? 2 : 0; }
 
+// Slices of a workgroup's busiest wave (without those rounds, which a shorter K does not have).
+inline int staged_most_slices(int waves, int k) {
+  const int slices = k / 64, rounds = slices / waves, rest = slices - rounds * waves;
+  return rounds + (rest + waves / 2 - 1) / (waves / 2);
+}
+
+// Four column tiles, up to 16 rows: four waves or eight.  Eight while there is one workgroup per compute unit at most, which a unit
+// with four waves only makes wait longer for its memory; four beyond, when a unit holds several small workgroups instead of a
+// second round of large ones, and where eight waves would not have fewer slices each.  The faster of the two on 336 of the
+// 338 shapes it decides out of 1563 (both blockings; none of the others by more than 2 %): M = 8, N = 18432, K = 4096 along N 12.9 with
+// four and 16.2 us with eight waves, M = 6, N = 14336, K = 1216 along K 5.4 and 4.6, M = 4, N = 13824, K = 256 along N 2.89 and 3.03.
+inline bool staged_four_waves(int n, int k) {
+  return (n / 16 + 3) / 4 > kComputeUnits || staged_most_slices(4, k) <= staged_most_slices(8, k);
+}
+
 // LDS of a workgroup: per wave `depth` slots of 16 * mt rows x 128 bytes, 32 columns of packed weights at a time, scales and
 // zero-points 256 bytes at a time; the waves' partial tiles take their place at the end.
 constexpr int staged_lds_bytes(bool row, int block_size, bool has_zp, int nt, int mt, int waves, int depth) {
@@ -362,9 +377,11 @@ inline int cost_form(bool column_wise, bool bf16, int block_size, bool has_zp) {
 // and row groups of 48.  A launch takes, in us, a fixed part, the packed weights' way from HBM, and rounds of workgroups as
 // the busiest XCD has them, each a fixed part and a part per 1024 k that grows with the rows and, per column tile, with the form.
 // Least squares over plans up to 1.4 times their shape's fastest, four fifths of them with the weights in HBM, every form: up
-// to 16 rows 15284 plans of 4800 shapes (N = 1024 ... 28672, K = 64 ... 16384; 5.8 % rms along K, 6.9 % along N), more rows 32072
-// plans of 9030 shapes (M = 17 ... 700; 5.2 - 5.9 %).  The shape with the smallest estimate takes 1.002 times the fastest one's time in the
-// mean (at most 1.23) with more than 16 rows, 1.01 (1.28) with fewer.
+// to 16 rows 20385 plans of 6100 shapes (N = 1024 ... 28672, along N 131072, K = 64 ... 16384; four tiles in the waves that
+// staged_four_waves() gives them; a plan counts less the further it is behind its shape's fastest, half at a fifth; 6.5 % rms along
+// K, 6.6 % along N), more rows 32072 plans of 9030 shapes (M = 17 ... 700; 5.2 - 5.9 %).  The shape with the smallest estimate takes
+// 1.002 times the fastest one's time in the mean (at most 1.23) with more than 16 rows, 1.006 (1.16) along K and 1.005 (1.20) along N
+// with fewer.
 struct StagedShapeCost {
   int depth, nt, waves;
   double round, per_k;
@@ -376,16 +393,16 @@ struct StagedFamily {
 };
 inline const StagedFamily& staged_family(bool row, int mt) {
   static constexpr StagedFamily kAlongK[3] = {
-      {2.273, 4.945, 0.585, 0.544, 0.051, 0.028, -0.036, -0.055, 9,
-       {{4, 1, 8, 0.609, 0.413}, {2, 1, 16, 0.821, 0.304}, {2, 2, 16, 0.897, 0.470}, {2, 3, 16, 1.064, 0.708}, {2, 4, 8, 0.976, 0.822},
-        {2, 5, 8, 1.148, 1.091}, {2, 6, 8, 1.209, 1.314}, {2, 7, 8, 1.403, 1.569}, {2, 4, 4, 0.703, 0.965}}},
+      {2.401, 2.500, 0.261, 0.555, 0.049, 0.042, -0.036, 0.046, 9,
+       {{4, 1, 8, 0.314, 0.406}, {2, 1, 16, 0.544, 0.292}, {2, 2, 16, 0.620, 0.438}, {2, 3, 16, 0.823, 0.665}, {2, 4, 8, 0.717, 0.763},
+        {2, 5, 8, 0.864, 1.074}, {2, 6, 8, 0.958, 1.304}, {2, 7, 8, 1.137, 1.562}, {2, 4, 4, 0.404, 0.801}}},
       {1.362, 3.678, 0.567, 0.418, 0.045, 0.036, -0.022, 0.031, 5,
        {{2, 1, 8, 1.302, 0.555}, {2, 2, 8, 1.419, 0.636}, {2, 4, 8, 1.949, 0.942}, {2, 6, 8, 2.441, 1.484}, {2, 8, 8, 2.739, 1.927}}},
       {1.210, 3.573, 0.721, 0.411, 0.039, 0.031, -0.032, 0.035, 5,
        {{2, 1, 8, 1.511, 0.608}, {2, 2, 8, 1.895, 0.779}, {2, 3, 8, 2.346, 0.973}, {2, 4, 8, 2.652, 1.145}, {2, 5, 8, 3.057, 1.477}}}};
   static constexpr StagedFamily kAlongN[3] = {
-      {2.142, 4.216, 1.064, 0.378, 0.141, 0.038, -0.062, -0.041, 5,
-       {{4, 1, 8, 0.732, 0.490}, {2, 1, 16, 1.000, 0.365}, {2, 2, 16, 1.098, 0.545}, {2, 4, 8, 1.067, 0.953}, {2, 4, 4, 0.779, 1.172}}},
+      {2.293, 2.893, 1.664, 0.398, 0.138, 0.016, -0.060, 0.004, 5,
+       {{4, 1, 8, 0.433, 0.497}, {2, 1, 16, 0.686, 0.375}, {2, 2, 16, 0.804, 0.550}, {2, 4, 8, 0.820, 0.940}, {2, 4, 4, 0.451, 0.979}}},
       {1.476, 3.494, -0.106, 0.373, 0.128, 0.072, -0.044, 0.028, 4,
        {{2, 1, 8, 1.293, 0.547}, {2, 2, 8, 1.566, 0.643}, {2, 4, 8, 1.985, 1.077}, {2, 8, 8, 2.768, 2.310}}},
       {1.404, 3.637, -0.203, 0.344, 0.125, 0.073, -0.043, 0.047, 3,
@@ -420,7 +437,7 @@ inline StreamingShape streaming_shape(bool row, int m, int n, int k, int block_s
     for (int i = 0; i < f.count; ++i) {
       const StagedShapeCost& c = f.shapes[i];
       if (!staged_shape_exists(row, block_size, (form & kCostNoZeroPoints) == 0, c.nt, mt, c.waves, c.depth)) continue;
-      if (mt == 1 && row && n >= 22528 && c.waves != 4) continue;
+      if (mt == 1 && c.nt == 4 && (c.waves == 4) != staged_four_waves(n, k)) continue;
       const double t = staged_estimate_us(f, c, m, n, k, row_groups, form);
       if (s.nt != 0 && t >= best) continue;
       best = t;
@@ -705,14 +722,16 @@ constexpr uint64_t kStreamingMaxWeights = uint64_t{1} << 33;
 
 // What the streaming kernel has to promise to take a shape from the decode kernel, in us; 0: it does not.  Blocks along N, where the
 // decode kernel has one column tile per workgroup: less than 0.92 of its own estimate (523 shapes, K up to 8192: 7.5 % rms;
-// M = 2, N = 28416, K = 7936 42.6 -> 25.2 us, M = 3, N = 27072, K = 1152 10.3 -> 6.6; one of 60 or so that change is more than 2 %
-// slower).  Blocks along K, K > 8192, where it needs sixteen waves, up to 28672 columns: less than its estimate (90 shapes, M = 4, N =
-// 10496, K = 8704 17.9 -> 13.2, M = 2, N = 7680, K = 8448 15.3 -> 11.7; 30 change, none is slower).
+// M = 2, N = 28416, K = 7936 42.6 -> 25.2 us, M = 3, N = 27072, K = 1152 10.3 -> 6.6), 0.87 up to K = 1152 (of 55 shapes there between
+// 0.87 and 0.92 of it 26 are faster and 18 slower by more than 2 %, below it 48 and 4; with a longer K 137 and 12).  Of 215 measured
+// shapes that it gives to the streaming kernel 185 are faster and 16 slower, 1.19 in the mean.  Blocks along K, K > 8192, where it
+// needs sixteen waves, up to 28672 columns: less than its estimate (90 shapes, M = 4, N = 10496, K = 8704 17.9 -> 13.2, M = 2, N = 7680,
+// K = 8448 15.3 -> 11.7).
 inline double decode_bar_us(const DecodeShape& d, int n, int k, int form) {
   const double kk = static_cast<double>(k) / 1024.0, t = static_cast<double>(n) / 4096.0;
   const double full = static_cast<double>((n + 4095) / 4096);
   const double bf = (form & kCostBf16) ? 1.0 : 0.0, no_zp = (form & kCostNoZeroPoints) ? 1.0 : 0.0, more = d.rows > 1 ? 1.0 : 0.0;
-  if (d.row != 0) return 0.92 * (2.522 + 0.155 * t + kk * (full * (0.337 + 0.048 * more) + t * (0.188 + 0.208 * bf - 0.213 * no_zp)));
+  if (d.row != 0) return (k <= 1152 ? 0.87 : 0.92) * (2.522 + 0.155 * t + kk * (full * (0.337 + 0.048 * more) + t * (0.188 + 0.208 * bf - 0.213 * no_zp)));
   if (d.waves == 16 && k > 8192 && n <= 28672) {
     return 1.777 + 2.259 * t + kk * (full * (0.345 + 0.060 * more) + t * (0.045 * bf - 0.022 * no_zp - 0.061));
   }
