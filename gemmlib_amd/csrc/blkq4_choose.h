@@ -428,6 +428,13 @@ inline double staged_estimate_us(const StagedFamily& f, const StagedShapeCost& c
 // most 6 %, all of them along K), and faster by a fifth in the mean along K (M = 16, N = 4224, K = 2624 9.7 -> 5.7 us, M = 2,
 // N = 13376, K = 5440 15.0 -> 10.1), by half along N (M = 11, N = 1536, K = 512 8.1 -> 3.2); in row groups, 113 shapes, it is
 // faster on all (1.09 - 2.25 times, M = 57, N = 6080, K = 1856 10.7 -> 9.3).
+//
+// Row groups of 48 only where they are fewer than groups of 32: as many of them are never faster along N (1422 shapes), and along K
+// on 29 of 1854 by 2 to 4 %, while their estimate, a twentieth off either way, chose them more often (253 drawn shapes: 113 are faster
+// in groups of 32 by more than 2 %, 23 slower; M = 23, N = 20480, K = 8128 27.4 -> 24.2 us).  A single group (33 to 48 rows) along K
+// that leaves an eighth of the compute units without a workgroup has to promise 4 % less than two groups of 32, whose workgroups
+// hold twice the columns (269 drawn shapes: 207 faster, 8 slower, 1.05 in the mean; M = 35, N = 6016, K = 5120 11.2 -> 10.3); with every
+// unit busy the estimates are level (M = 34, N = 8192, K = 4096 9.3 us, two groups of 32 11.2).
 inline StreamingShape streaming_shape(bool row, int m, int n, int k, int block_size, int form, double* us) {
   StreamingShape s{};
   double best = 0.0;
@@ -438,9 +445,14 @@ inline StreamingShape streaming_shape(bool row, int m, int n, int k, int block_s
       const StagedShapeCost& c = f.shapes[i];
       if (!staged_shape_exists(row, block_size, (form & kCostNoZeroPoints) == 0, c.nt, mt, c.waves, c.depth)) continue;
       if (mt == 1 && c.nt == 4 && (c.waves == 4) != staged_four_waves(n, k)) continue;
+      if (mt == 3 && row_groups == (m + 31) / 32) continue;
       const double t = staged_estimate_us(f, c, m, n, k, row_groups, form);
-      if (s.nt != 0 && t >= best) continue;
-      best = t;
+      const bool one_group_bar = mt == 3 && row_groups == 1 && !row &&
+                                 streaming_busiest_xcd(1, (n / 16 + c.nt - 1) / c.nt, streaming_neighbours(c.nt, c.waves, c.waves)) < 28;
+      const double price = one_group_bar ? 1.04 * t : t;
+      if (s.nt != 0 && price >= best) continue;
+      best = price;
+      *us = t;
       s.depth = c.depth; s.nt = c.nt; s.mt = mt; s.waves = c.waves; s.am = kRowsPerSlotInLds; s.split = c.waves;
       s.row_groups = row_groups;
     }
@@ -474,7 +486,6 @@ inline StreamingShape streaming_shape(bool row, int m, int n, int k, int block_s
     }
   }
   streaming_geometry(&s, row, n, k);
-  *us = best;
   return s;
 }
 
