@@ -485,11 +485,12 @@ inline StreamingShape streaming_shape(bool row, int m, int n, int k, int block_s
       }
     }
   }
-  // A single row group of 48 along K in two or more rounds of workgroups takes 8 % longer than its estimate where that lies near the one
-  // of 64 x 128 tiles, 160 to 190 of which cover those layers (38 drawn shapes change for it: 25 are faster by more than 2 %, 4 slower,
-  // 1.03 in the mean; M = 46, N = 20992, K = 7744, bf16 38.2 -> 35.1 us, M = 47, N = 22976, K = 3456 20.4 -> 18.7).
+  // A single row group of 48 along K in two rounds of workgroups takes 8 % longer than its estimate where that lies near the one
+  // of 64 x 128 tiles, 160 to 190 of which cover those layers (59 drawn shapes change for it: 40 are faster by more than 2 %, 9 slower,
+  // 1.03 in the mean; M = 46, N = 20992, K = 7744, bf16 38.2 -> 35.1 us, M = 47, N = 22976, K = 3456 20.4 -> 18.7).  In more rounds
+  // either may be ahead (24 shapes: 9 and 7; M = 33, N = 45120, K = 3008, bf16 is 7 % faster than tiles).
   if (s.mt == 3 && !row && s.row_groups == 1 &&
-      streaming_rounds(1, (n / 16 + s.nt - 1) / s.nt, streaming_neighbours(s.nt, s.waves, s.split)) > 1) {
+      streaming_rounds(1, (n / 16 + s.nt - 1) / s.nt, streaming_neighbours(s.nt, s.waves, s.split)) == 2) {
     *us *= 1.08;
   }
   streaming_geometry(&s, row, n, k);
