@@ -1,5 +1,6 @@
 // Weight-streaming kernel for gfx950, rows whole in LDS.  It starts by name only (blkq4_gemm_with_plan_sm80): with rows staged slice by
-// slice (blkq4_staged.hip) every shape that it ran is faster or level (measured beside streaming_shape() in blkq4_choose.h).
+// slice (blkq4_staged.hip) every shape that it ran is faster or level (measured beside streaming_shape() in blkq4_choose.h).  It is
+// kept because a plan's text is an interface: a text that a program noted down ("streaming ... 1 ...") starts the kernel it names.
 //
 // The work is a stream over the packed weights (K*N/2 bytes plus scales and zero-points) that has to
 // run at HBM speed; everything else is arranged so that the stream is requested as early and as
@@ -605,9 +606,8 @@ int launch_kernel(const blkq4_gemm_args* a) {
   }
 }
 
-// The shapes that exist, (DEPTH, NT, MT, waves, split): what blkq4::choose() may ask for, and, blocks along K in row groups of
-// 32, what only a plan given by name starts (choose() has their rows staged per slice).  Blocks along N:
-// those with one column tile per wave (28 registers of packed weights, scales and zero-points per slot and tile).
+// The shapes that exist, (DEPTH, NT, MT, waves, split): what a plan may name.  Blocks along N: those with one column tile per wave
+// (28 registers of packed weights, scales and zero-points per slot and tile).
 #define BLKQ4_STREAMING_SHAPES(X)                                                                          \
   /* row groups of 32 */                                                                                   \
   X(2, 1, 2, 8, 8) X(2, 2, 2, 8, 8) X(2, 4, 2, 8, 8) X(2, 6, 2, 8, 8) X(2, 8, 2, 8, 8)                     \
