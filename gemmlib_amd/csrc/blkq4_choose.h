@@ -314,7 +314,7 @@ constexpr int staged_lds_bytes(bool row, int block_size, bool has_zp, int nt, in
 }
 
 // Blocks along N: one, two, four or eight column tiles (whole column groups, or a part of one).
-// Five tiles of 48 rows fit where there are at most two block rows to a slice.
+// Five tiles of 48 rows fit in LDS unless a slice has four block rows of scales and of zero-points (blocks of 16 with them).
 constexpr bool staged_shape_exists(bool row, int block_size, bool has_zp, int nt, int mt, int waves, int depth) {
   if (row && nt != 1 && nt != 2 && nt != 4 && nt != 8) return false;
   return static_cast<size_t>(staged_lds_bytes(row, block_size, has_zp, nt, mt, waves, depth)) <= kMaxLdsBytes;
