@@ -15,12 +15,12 @@
 //     its four words), which keeps the slice 64 deep.  64 because K is a multiple of that: there is no partial slice.
 //   - Row groups of 48: 33 to 48 rows are one group instead of two, so every weight is fetched and converted once: 40 rows,
 //     N = 14336, K = 4096 16.9 -> 13.0 us, M = 48, N = 11008 14.7 -> 12.7, M = 144, N = 4096 12.9 -> 12.1.  (64 rows a group
-//     were no faster on any shape tried: M = 64, N = 8192 11.1 in two groups, 12.4 in one.)
+//     were tried on one shape, along K: M = 64, N = 8192, K = 4096 11.1 in two groups, 12.4 in one.)
 //   - Blocks along N: with one column tile a workgroup fetches the rows again for every 16 columns and builds the zero-point
 //     constants of its 16-row groups (half of a word's instructions) for one tile.  Two, four or eight tiles share both: K = N = 4096,
 //     M = 150 11.7 us (tiles, which ran there, 16.3), M = 48, N = 8192, K = 2048 11.7 -> 7.0, M = 12, N = 53440, K = 3584 45.5 -> 28.8.
 //   - The copies' lane offsets never change, the slice moves a scalar base: a request costs no vector instruction.
-//   - Rows are dealt evenly to the row groups (48 rows: two groups of 24); the row groups of a column group run on one
+//   - Rows are dealt evenly to the row groups (64 rows: two groups of 32); the row groups of a column group run on one
 //     XCD and share its weights there.  With a single row group the weights are read once per launch: non-temporal.
 //   - A SIMD serves its older wave first, also its memory requests: of eight waves the younger four get their first slice
 //     1.8 us after the others (M = 48, N = 11008) and finish last.  So the older half takes extra rounds of slices
@@ -148,13 +148,10 @@ __global__ __launch_bounds__(64 * kWaves)
 
   // Workgroup -> (row group, column group), as streaming_geometry() deals them: workgroup w runs on XCD w % 8, an XCD takes
   // the row groups of a column group, then the next of a few neighbouring column groups.
-  // (q / row_groups by a multiplication: the division takes 30 instructions in front of the first request, and is left to
-  // grids so large that the multiplication is not exact)
+  // (q / row_groups by a multiplication: the division takes 30 instructions in front of the first request)
   const int col_groups = static_cast<uint32_t>(N + L::kCols - 1) / L::kCols;
   const uint32_t q = blockIdx.x >> 3;
-  const uint32_t cq = row_groups == 1       ? q
-                      : row_groups_inv != 0 ? __umulhi(q, row_groups_inv)
-                                            : q / static_cast<uint32_t>(row_groups);
+  const uint32_t cq = row_groups == 1 ? q : __umulhi(q, row_groups_inv);
   const uint32_t rg = q - cq * row_groups;
   constexpr int kNeighbours = streaming_neighbours(NT, kWaves, kWaves);
   const int cg = kNeighbours * ((blockIdx.x & 7) + 8 * (cq / kNeighbours)) + (cq % kNeighbours);
@@ -435,11 +432,12 @@ int launch_kernel(const blkq4_gemm_args* a) {
       p.grid != static_cast<uint32_t>(p.cg_stride) * static_cast<uint32_t>(p.row_groups)) {
     return static_cast<int>(hipErrorInvalidValue);
   }
-  // q / row_groups = (q * inv) >> 32 with inv = floor(2^32 / row_groups) + 1: exact while q * row_groups < 2^32 (inv *
-  // row_groups is at most row_groups over 2^32), q below the workgroups of an XCD.  0: the kernel divides.
+  // q / row_groups = (q * inv) >> 32 with inv = floor(2^32 / row_groups) + 1 (unused with one row group): exact while q *
+  // row_groups < 2^32 (inv * row_groups is at most row_groups over 2^32), q below the workgroups of an XCD.  At most 32 row
+  // groups of weights below 4 GiB, K from 64 on, come to 2^30.
   const uint64_t groups = static_cast<uint32_t>(p.row_groups);
-  const uint32_t row_groups_inv =
-      (p.grid >> 3) * groups < (uint64_t{1} << 32) ? static_cast<uint32_t>((uint64_t{1} << 32) / groups + 1) : 0;
+  if ((p.grid >> 3) * groups >= (uint64_t{1} << 32)) return static_cast<int>(hipErrorInvalidValue);
+  const uint32_t row_groups_inv = static_cast<uint32_t>((uint64_t{1} << 32) / groups + 1);
   if (a->dry_run) return 0;  // the plan has passed every check a launch makes
   constexpr auto kernel = staged_mfma_kernel<BS, HAS_ZP, NT, MT, kWaves, DEPTH, ROW>;
   const hipError_t attr = raise_lds_limit_once(reinterpret_cast<const void*>(kernel), kMaxLdsBytes, &lds_limit_flags<kernel>());
