@@ -424,10 +424,10 @@ inline double staged_estimate_us(const StagedFamily& f, const StagedShapeCost& c
 
 // The streaming kernel's shape for any number of rows, and what it is expected to take: the smallest estimate of all shapes with rows
 // staged per slice.  Rows whole in LDS (blkq4_skinny.hip), which used to run up to 16 rows and some row groups with blocks
-// along N, start by name only: of 2156 shapes of up to 16 rows that took them the shape chosen here is slower by more than 2 % on 16 (at
-// most 6 %, all of them along K), and faster by a fifth in the mean along K (M = 16, N = 4224, K = 2624 9.7 -> 5.7 us, M = 2,
-// N = 13376, K = 5440 15.0 -> 10.1), by half along N (M = 11, N = 1536, K = 512 8.1 -> 3.2); in row groups, 113 shapes, it is
-// faster on all (1.09 - 2.25 times, M = 57, N = 6080, K = 1856 10.7 -> 9.3).
+// along N, start by name only: timed in turn on 715 drawn shapes of up to 16 rows that took them (70 of them with 28736 to 131072
+// columns) the shape chosen here is slower by more than 2 % on none; along K it is 1.25 times as fast in the mean (M = 16, N = 4224, K = 2624
+// 9.7 -> 5.7 us, M = 2, N = 13376, K = 5440 15.0 -> 10.1), along N 1.63 times (M = 11, N = 1536, K = 512 8.1 -> 3.2); in row groups,
+// 113 shapes, it is faster on all (1.09 - 2.25 times, M = 57, N = 6080, K = 1856 10.7 -> 9.3).
 //
 // Row groups of 48 only where they are fewer than groups of 32: as many of them are never faster along N (1422 shapes), and along K
 // on 29 of 1854 by 2 to 4 %, while their estimate, a twentieth off either way, chose them more often (253 drawn shapes: 113 are faster
@@ -745,7 +745,9 @@ constexpr uint64_t kStreamingMaxWeights = uint64_t{1} << 33;
 // 0.87 and 0.92 of it 26 are faster and 18 slower by more than 2 %, below it 48 and 4; with a longer K 137 and 12).  Of 215 measured
 // shapes that it gives to the streaming kernel 185 are faster and 16 slower, 1.19 in the mean.  Blocks along K, K > 8192, where it
 // needs sixteen waves, up to 28672 columns: less than its estimate (90 shapes, M = 4, N = 10496, K = 8704 17.9 -> 13.2, M = 2, N = 7680,
-// K = 8448 15.3 -> 11.7).
+// K = 8448 15.3 -> 11.7).  On wider layers, which neither estimate was fitted on, whatever decode_shape() takes stays with the decode
+// kernel, although it is behind on most: of 84 shapes with N = 28736 ... 57344, K = 8448 ... 16384 the streaming kernel is faster on 81,
+// by 1.02 to 1.73 times with two to four rows, with one row from 0.88 to 1.53.
 inline double decode_bar_us(const DecodeShape& d, int n, int k, int form) {
   const double kk = static_cast<double>(k) / 1024.0, t = static_cast<double>(n) / 4096.0;
   const double full = static_cast<double>((n + 4095) / 4096);

@@ -35,12 +35,13 @@
 //   M = 16, N = 28672, K = 8192    5.1, 22.4, 22.4   25.5   the weight stream, 5.9 TB/s; the rows cost nothing beside it
 //   M = 12, N = 128256, K = 4096   10.9, 46.5, 50.0  54.7   the same
 //   M = 48, N = 11008, K = 4096    5.2, 9.0, 11.5    14.0   two groups of 24 rows: rows and weights overlap in part; conversion,
-//                                                           twice per weight (one group of 48 rows: -, 7.2, 11.6, 12.7)
+//                                                           twice per weight (one group of 48 rows: -, 7.2, 11.6, 13.1)
 //   M = 128, N = K = 4096          4.9, 5.0, 7.1     8.9    the same, four times per weight
-// Why rows and weights do not overlap better: a compute unit's vector cache returns what it was asked for in order, and what is
-// asked for occupies its 32 KB until then.  Rows alone, or weights that lie in L2, come at 120 - 130 bytes a ns (64 a cycle); with
-// weights from HBM (950 cycles, L2 236) between them everything comes at 32 KB per HBM answer, about 70 bytes a ns, whatever the
-// order of the slices over the workgroups, and also when the rows have been brought into every L2 beforehand (both tried).
+// Why rows and weights do not overlap better, as far as it is understood: a compute unit's vector cache returns what it was asked for
+// in order, and what is asked for occupies its 32 KB until then.  Rows alone, or weights that lie in L2, come at 126 - 150 bytes a ns
+// (64 a cycle); with weights from HBM (950 cycles, L2 236) between them 32 KB per HBM answer would be 70 bytes a ns; 48 rows
+// see 53, whatever the order of the slices over the workgroups, and also when the rows have been brought into every L2 beforehand
+// (both tried).
 // What the conversion adds shares its issue port with the MFMAs, at 1.6 (M = 512) to 2.0 GHz (M = 48): the chip is power limited.
 // fp16, blocks of 64, K = 4096, us, against the kernel before (128-deep slices, weights in registers, refilled after use), a few
 // weight sets in turn that the Infinity Cache holds:
