@@ -141,8 +141,9 @@ inline uint32_t decode_grid(int n, int nt) {
 //   - one to four rows, K > 8192 (where the decode kernel needs sixteen waves), 832 to 1792 column tiles (M = 1:
 //     K = 16384, N = 28672 51.1 -> 45.5 us, N = 13312 29.7 -> 25.1; K = N = 28672 87.0 -> 75.8; K = 8256, N = 13312 18.4 ->
 //     14.9; K = 11008, N = 28672 with zero-points 42.6 -> 37.7, N = 14336 without 19.0 -> 20.6, the one loss found; on
-//     wider layers the decode kernel is ahead again: K = 11008, N = 36864 41.4 against 44.0).
-// At K = 4096 and on wider layers the decode kernel wins.
+//     wider layers the decode kernel was ahead again: K = 11008, N = 36864 41.4 against 44.0).
+// At K = 4096 and on wider layers the decode kernel won.  (Both against the streaming kernel of that time; what today's promises is
+// weighed in decode_bar_us().)
 // (The first case later, against the decode kernel's eight waves with eight slices each and one tile per workgroup:
 // with blocks of 32 or 64 two and three rows are 2 - 7 % faster in the decode kernel up to 1792 tiles -- M = 2, K = 8192,
 // N = 22016 21.3 against 23.0 us, N = 28672 26.0 against 27.7 -- four rows level, N = 57344 level to 8 % behind; with blocks
